@@ -39,6 +39,7 @@ FLAGS = [
 def sources(lmax: int = LMAX) -> list[Path]:
     classes = builder_classes(lmax)
     files = gen_hip.generate(classes)
+    files += gen_hip.generate_coop(classes)   # the quartet-cooperative F kernels
     # the classes with an f shell: entries onto the loop-form fused kernel
     loop = [c for c in builder_classes(LOOP_LMAX) if max(c) > lmax]
     if loop:
@@ -49,6 +50,7 @@ def sources(lmax: int = LMAX) -> list[Path]:
         files.append(p)
     built = set(classes) | set(loop)
     gen_hip.write_header(tuple(c for c in builder_classes(LOOP_LMAX) if c in built))
+    gen_hip.write_coop_header(classes)
     p = gen_hip.GEN / "f_any_table.h"
     text = gen_hip.emit_any_table(tuple(c for c in builder_classes(LOOP_LMAX) if c in built))
     if not p.exists() or p.read_text() != text:
@@ -72,9 +74,11 @@ def _compile(src: Path, extra: list[str], force: bool = False) -> tuple[Path, fl
     obj = OBJ / (src.stem + ".o")
     deps = [src, CSRC / "fj_device.h", HERE.parent / "include" / "fj_mi355x.h",
             CSRC / "gen" / "fj_boys_table.h"]
-    hdr = src.parent / (src.stem.replace("_r32", "") + ".h")
+    hdr = src.parent / (src.stem.replace("_r32", "").replace("_mx", "") + ".h")
     if hdr.exists():
         deps.append(hdr)
+    if src.name.startswith("c_"):
+        deps.append(CSRC / "fj_coop.h")
     if src.name in ("fj_kloop.hip", "fj_dfloop.hip", "fj_gfloop.hip"):
         deps.append(CSRC / "fj_kloop.h")
     if src.name == "fj_gfloop.hip":

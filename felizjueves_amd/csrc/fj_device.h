@@ -89,6 +89,13 @@ __device__ __forceinline__ fj_v4d fj_mfma_f64_16x16x4(double a, double b, fj_v4d
 // values derived from them are recomputed after it, not hoisted above it.
 #define FJ_LAUNDER(p, s) __asm__ volatile("" : "+v"(p), "+s"(s))
 
+// Orders the LDS accesses of a wavefront's lanes before and after it (the
+// wavefront issues them in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void fj_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // First primitive record and degree of pair i of one side.
 __device__ __forceinline__ void fj_side_range(const FjSide& s, int i, int& k0, int& k) {
     if (s.off) {

@@ -126,6 +126,45 @@ class Launch:
     n_quartets32: int = 0     # MIXED: the FP32 items' quartets (as planned)
     n_cold: int = 0           # the last n_cold FP64 items hold the cold kets (see COLD)
     tier_dev: object = None   # MIXED: per-item tiers chosen on the device per build
+    coop: object = None       # the launch's CoopItems when it runs quartet-cooperatively
+
+
+@dataclass
+class CoopItems:
+    """A launch's items for the quartet-cooperative kernel: whole kets, at
+    most a batch per item; parent the planned item each comes from."""
+    work: np.ndarray          # [n, 4] int32 (bra, first list entry, system, end entry)
+    ket_list: np.ndarray
+    parent: np.ndarray
+    parts: int
+    dev: tuple = ()           # (work, ket_list, parent) on the device
+
+
+def coop_items(work: np.ndarray, ket_list: np.ndarray, batch: int):
+    """(work, ket list, parent) of planned items for the cooperative kernel.
+    Of a planned item's lanes (ket, primitive chunk) the ones with a first
+    chunk name its kets, and of the items of one bra pair's chunks the first
+    lists every lane, so each quartet of the plan is taken once, whole. An
+    item's kets are cut into equal pieces of at most `batch`."""
+    first = (ket_list & (0x7f << 17)) == 0
+    at = np.zeros(len(ket_list) + 1, dtype=np.int64)
+    np.cumsum(first, out=at[1:])
+    w = work.astype(np.int64)
+    parent = np.nonzero(((w[:, 2] >> 16) & 0xff) == 0)[0]
+    k0, n = at[w[parent, 1]], at[w[parent, 3]] - at[w[parent, 1]]
+    pieces = -(-n // batch)
+    rep = np.repeat(np.arange(len(parent)), pieces)
+    j = np.arange(len(rep)) - np.repeat(np.cumsum(pieces) - pieces, pieces)
+    lo = k0[rep] + j * n[rep] // pieces[rep]
+    hi = k0[rep] + (j + 1) * n[rep] // pieces[rep]
+    out = np.stack([w[parent[rep], 0], lo, w[parent[rep], 2] & 0xffff, hi], axis=1)
+    return out.astype(np.int32), (ket_list[first] & 0x1ffff).astype(np.int32), parent[rep].astype(np.int32)
+
+
+# Workgroups a cooperative launch aims for: an item's primitive quartets are
+# shared by several while there are fewer items (a CU holds one to four, and
+# the items' costs differ).
+COOP_GROUPS = 1024
 
 
 WAVE = 64             # lanes of a wavefront
@@ -285,11 +324,11 @@ class FockBuilder:
     def __init__(self, basis: Basis, D: np.ndarray, *, tau: float = 1e-12, threads=64,
                  mixed: bool = False, fp32_error: float = 1e-11, selector=None,
                  lane_flops=None, fp32_bound: float | None = None, planner: str = "auto",
-                 merge_tiers: bool = True, orient: bool = True, fp32_classes=None):
+                 merge_tiers: bool = True, orient: bool = True, fp32_classes=None, coop=None):
         self._setup([(basis, D)], tau=tau, threads=threads, mixed=mixed, fp32_error=fp32_error,
                      selector=selector, lane_flops=lane_flops, fp32_bound=fp32_bound,
                      planner=planner, merge_tiers=merge_tiers, orient=orient,
-                     fp32_classes=fp32_classes)
+                     fp32_classes=fp32_classes, coop=coop)
 
     @classmethod
     def batch(cls, systems, **kw) -> "FockBuilder":
@@ -303,7 +342,7 @@ class FockBuilder:
     def _setup(self, systems, *, tau: float = 1e-12, threads=64, mixed: bool = False,
                fp32_error: float = 1e-11, selector=None, lane_flops=None,
                fp32_bound: float | None = None, planner: str = "auto",
-               merge_tiers: bool = True, orient: bool = True, fp32_classes=None):
+               merge_tiers: bool = True, orient: bool = True, fp32_classes=None, coop=None):
         """threads, lane_flops: one value for every class pair, or a dict
         {(la, lb, lc, ld): value} (the autotuner's choice per class pair;
         missing ones take the default 64 and the automatic split).
@@ -322,7 +361,15 @@ class FockBuilder:
         fp32_classes: the class pairs (la, lb, lc, ld) a mixed build may
         send to the FP32 tier (the autotuner's choice: where the mixed
         launch is measured faster than the FP64 one); the others run FP64
-        launches. None: every class pair."""
+        launches. None: every class pair.
+        coop: whether a launch runs in the quartet-cooperative form
+        (fj_fc_*; classes through d). None: every one, except a class pair
+        whose threads or lane_flops are given (they shape the per-lane
+        form). True / False: every class pair that has it / none. Measured,
+        one stream / four, per-lane -> cooperative: the three-atom s,s,p,d
+        system 26 -> 1.6 / 15.8 -> 0.5 ms, 9 atoms 31 -> 3.1 / 9.6 -> 1.7 ms,
+        40 atoms 104 -> 67 / 75 -> 66 ms."""
+        self.coop = coop
         self.merge_tiers = bool(merge_tiers)
         self.orient = bool(orient)
         self.fp32_classes = None if fp32_classes is None else {tuple(int(x) for x in c)
@@ -692,8 +739,9 @@ class FockBuilder:
         for t in self.tables.values():
             t.dev["amp"] = native.to_dev(np.asarray(t.amp, dtype=np.float64))
         for L in self.launches:
-            L.work_dev = native.to_dev(L.work)
-            L.ket_list_dev = native.to_dev(L.ket_list)
+            L.coop = self._coop(L)
+            if L.coop is None or L.precision == MIXED:   # else no launch reads the per-lane lists
+                self.per_lane(L)
             if self.mixed and L.precision == MIXED:
                 self._tier_setup(L)
         # per system: shell offsets/sizes, Dsh and F (views of flat buffers)
@@ -714,6 +762,33 @@ class FockBuilder:
         self.F, self.Dsh = self.Fs[0], self.Dshs[0]
         self._sys_for = None
         self._dev = True
+
+    def per_lane(self, L: "Launch"):
+        """(work, ket list) of a launch's planned per-lane items on the device."""
+        if L.work_dev is None:
+            L.work_dev = native.to_dev(L.work)
+            L.ket_list_dev = native.to_dev(L.ket_list)
+        return L.work_dev, L.ket_list_dev
+
+    def _coop(self, L: "Launch"):
+        """The launch's items for the cooperative kernel, or None when it
+        keeps the per-lane form."""
+        batch = native.coop_batch(L.cls)
+        shaped = (self.lane_flops is not None or self.threads != 64 or L.cls in self.class_threads
+                  or L.cls in self.class_lane_flops)
+        if not batch or L.precision == FP32 or self.coop is False or (self.coop is None and shaped):
+            return None
+        work, kets, parent = coop_items(L.work, L.ket_list, batch)
+        if not len(work):
+            return None
+        # share the primitive quartets of an item over more workgroups while
+        # there are few items and each has full passes to give
+        deg = np.concatenate([[0], np.cumsum(L.ket.deg[kets])])
+        most = int((L.bra.deg[work[:, 0]] * (deg[work[:, 3]] - deg[work[:, 1]])).max())
+        parts = max(1, min(COOP_GROUPS // len(work), -(-most // 256), 64))
+        c = CoopItems(work, kets, parent, parts)
+        c.dev = tuple(native.to_dev(x) for x in (work, kets, parent))
+        return c
 
     def _tier_setup(self, L: "Launch") -> None:
         """The device side of a mixed launch's per-build tier choice: the
@@ -786,13 +861,19 @@ class FockBuilder:
         if ws is None:
             ws = self._ws = []
         need = min(WS_MAX_BYTES, max([native.workspace_bytes(L.cls, L.threads, L.work.shape[0])
-                                      for L in self.launches] + [0]))
+                                      for L in self.launches if L.coop is None] + [0]))
         while len(ws) <= i:
             ws.append(torch.empty(need // 8, dtype=torch.float64, device=native.device())
                       if need else None)
         return ws[i]
 
     def launch(self, L: "Launch", sys, stream=None, ws=None) -> None:
+        if L.coop is not None:
+            c = L.coop
+            native.call_fc(L.cls, c.parts, L.bra.side, L.ket.side, c.dev[0], c.work.shape[0], c.dev[1],
+                           c.dev[2], L.tier_dev if L.precision == MIXED else None, sys, L.diag,
+                           self.tau, stream)
+            return
         if L.precision == MIXED:
             native.call_fxm(L.cls, L.threads, L.bra.side, L.ket.side, L.work_dev, L.work.shape[0],
                             L.n_fp64, sys, L.diag, self.tau, stream, L.ket_list_dev, ws,

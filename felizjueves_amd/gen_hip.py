@@ -102,6 +102,83 @@ def _fidx_out(split: bool, r: str, c: str) -> str:
     return f"({r}) * dg.fr + ({c}) * dg.fc" if split else f"({r}) * n_ao + {c}"
 
 
+def _vrr_factors(v, nodes) -> set:
+    """The quartet factors the VRR statements of `nodes` read: (factor, axis)
+    for the vectors, (factor, None) for the scalars."""
+    used = set()
+    for n in nodes:
+        r = v.terms[n]
+        if r:
+            d, ts = r
+            for t in ts:
+                used.add((t.coef, d if t.coef in ("PA", "WP", "QC", "WQ") else None))
+    return used
+
+
+def _emit_ket_prim(E: "_Emit", used, ind: int) -> None:
+    """A ket primitive pair's values, from its record q_."""
+    E("const double Qx = q_[0], Qy = q_[1], Qz = q_[2], q = q_[6], Uq = q_[7];", ind)
+    for d in range(3):
+        if ("QC", d) in used:
+            E(f"const R QC{AX[d]} = R(q_[{3 + d}]);", ind)
+    if ("i2q", None) in used or ("i2q_r", None) in used:
+        E("const double iq = 1.0 / q;", ind)
+
+
+def _emit_prim_vrr(E: "_Emit", v, L: int, nodes, used, boys: str, ind: int) -> None:
+    """A primitive quartet's scalars from its bra record p_ and the ket
+    values, and the VRR statements of `nodes` in build order."""
+    need = lambda c: (c, None) in used  # noqa: E731
+    E("const double PQx = p_[0] - Qx, PQy = p_[1] - Qy, PQz = p_[2] - Qz;", ind)
+    E("const double p = p_[6];", ind)
+    E("const double ippq = 1.0 / (p + q);", ind)
+    E("const double rho = p * q * ippq;", ind)
+    E("const double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);", ind)
+    E(f"double Fm[{L + 1}];", ind)
+    E(boys, ind)
+    E("const double S = p_[7] * Uq * (FJ_TWO_OVER_SQRT_PI * sqrt(rho));", ind)
+    for d in range(3):
+        if ("PA", d) in used:
+            E(f"const R PA{AX[d]} = R(p_[{3 + d}]);", ind)
+        if ("WP", d) in used:
+            E(f"const R WP{AX[d]} = R(-q * ippq * PQ{AX[d]});", ind)
+        if ("WQ", d) in used:
+            E(f"const R WQ{AX[d]} = R(p * ippq * PQ{AX[d]});", ind)
+    if need("i2p"):
+        E("const R i2p = R(0.5 * p_[8]);", ind)
+    if need("i2p_r"):
+        E("const R i2p_r = R(0.5 * p_[8] * rho * p_[8]);", ind)
+    if need("i2q"):
+        E("const R i2q = R(0.5 * iq);", ind)
+    if need("i2q_r"):
+        E("const R i2q_r = R(0.5 * iq * rho * iq);", ind)
+    if need("i2pq"):
+        E("const R i2pq = R(0.5 * ippq);", ind)
+    for n in v.order:
+        if n not in nodes:
+            continue
+        r = v.terms[n]
+        if not r:
+            E(f"const R {_vname(n)} = R(S * Fm[{n[2]}]);", ind)
+            continue
+        d, ts = r
+        parts = []
+        for t in ts:
+            c = t.coef
+            ch = _vname(t.child)
+            if c in ("PA", "WP", "QC", "WQ"):
+                parts.append(f"{c}{AX[d]} * {ch}")
+            else:
+                m = t.mult
+                sign = "-" if m < 0 else "+"
+                f = c if abs(m) == 1 else f"(R({abs(m)}) * {c})"
+                parts.append(f"{sign} {f} * {ch}")
+        expr = parts[0]
+        for p in parts[1:]:
+            expr += (" " + p) if p[0] in "+-" else (" + " + p)
+        E(f"const R {_vname(n)} = {expr};", ind)
+
+
 def emit_quartet(cls, split: bool = False) -> str:
     """The device function for one contracted quartet of class `cls`
     (split: the one-block digestion of the split J / K kernels, fj_qs_)."""
@@ -111,15 +188,7 @@ def emit_quartet(cls, split: bool = False) -> str:
     order, terms, targets, boundary = hrr_dag(tuple(cls))
     name = cls_name(cls)
     na, nb, nc, nd = (n_cart(x) for x in cls)
-    # which quartet factors the VRR reads
-    used = set()
-    for n in v.order:
-        r = v.terms[n]
-        if r:
-            d, ts = r
-            for t in ts:
-                used.add((t.coef, d if t.coef in ("PA", "WP", "QC", "WQ") else None))
-    need = lambda c: any(u[0] == c for u in used)  # noqa: E731
+    used = _vrr_factors(v, v.order)   # the quartet factors the VRR reads
     hrr_bra = any(r and r[0] == "bra" for r in terms.values())
     hrr_ket = any(r and r[0] == "ket" for r in terms.values())
     acc = {ef: f"c{i}" for i, ef in enumerate(v.targets)}
@@ -142,62 +211,10 @@ def emit_quartet(cls, split: bool = False) -> str:
         E(f"R c{i} = R(0);")
     E("for (int kc = 0; kc < k_cd; ++kc) {")
     E("const double* __restrict__ q_ = kp + 8 * kc;", 2)
-    E("const double Qx = q_[0], Qy = q_[1], Qz = q_[2], q = q_[6], Uq = q_[7];", 2)
-    for d in range(3):
-        if ("QC", d) in used:
-            E(f"const R QC{AX[d]} = R(q_[{3 + d}]);", 2)
-    if need("i2q") or need("i2q_r"):
-        E("const double iq = 1.0 / q;", 2)
+    _emit_ket_prim(E, used, 2)
     E("for (int kb = 0; kb < k_ab; ++kb) {", 2)
     E("const double* __restrict__ p_ = bp + FJ_SREC * kb;", 3)
-    E("const double PQx = p_[0] - Qx, PQy = p_[1] - Qy, PQz = p_[2] - Qz;", 3)
-    E("const double p = p_[6];", 3)
-    E("const double ippq = 1.0 / (p + q);", 3)
-    E("const double rho = p * q * ippq;", 3)
-    E("const double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);", 3)
-    E(f"double Fm[{L + 1}];", 3)
-    E(f"fj_boys<{L}>(T, Fm);", 3)
-    E("const double S = p_[7] * Uq * (FJ_TWO_OVER_SQRT_PI * sqrt(rho));", 3)
-    for d in range(3):
-        if ("PA", d) in used:
-            E(f"const R PA{AX[d]} = R(p_[{3 + d}]);", 3)
-        if ("WP", d) in used:
-            E(f"const R WP{AX[d]} = R(-q * ippq * PQ{AX[d]});", 3)
-        if ("WQ", d) in used:
-            E(f"const R WQ{AX[d]} = R(p * ippq * PQ{AX[d]});", 3)
-    if need("i2p"):
-        E("const R i2p = R(0.5 * p_[8]);", 3)
-    if need("i2p_r"):
-        E("const R i2p_r = R(0.5 * p_[8] * rho * p_[8]);", 3)
-    if need("i2q"):
-        E("const R i2q = R(0.5 * iq);", 3)
-    if need("i2q_r"):
-        E("const R i2q_r = R(0.5 * iq * rho * iq);", 3)
-    if need("i2pq"):
-        E("const R i2pq = R(0.5 * ippq);", 3)
-    # VRR, in build order
-    for n in v.order:
-        r = v.terms[n]
-        if not r:
-            E(f"const R {_vname(n)} = R(S * Fm[{n[2]}]);", 3)
-            continue
-        d, ts = r
-        parts = []
-        for t in ts:
-            c = t.coef
-            ch = _vname(t.child)
-            if c in ("PA", "WP", "QC", "WQ"):
-                parts.append(f"{c}{AX[d]} * {ch}")
-            else:
-                m = t.mult
-                sign = "-" if m < 0 else "+"
-                mag = abs(m)
-                f = c if mag == 1 else f"(R({mag}) * {c})"
-                parts.append(f"{sign} {f} * {ch}")
-        expr = parts[0]
-        for p in parts[1:]:
-            expr += (" " + p) if p[0] in "+-" else (" + " + p)
-        E(f"const R {_vname(n)} = {expr};", 3)
+    _emit_prim_vrr(E, v, L, v.order, used, f"fj_boys<{L}>(T, Fm);", 3)
     for ef, cname in acc.items():
         E(f"{cname} += {_vname((ef[0], ef[1], 0))};", 3)
     E("}", 2)
@@ -1318,75 +1335,17 @@ def emit_quartet_staged(cls, split: bool = False) -> str:
         """The primitive nest of one group: its accumulators, the closure of
         its targets, the contracted values stored to the boundary."""
         nodes = closure(v, [(e, f, 0) for e, f in tg])
-        used = set()
-        for n in nodes:
-            r = v.terms[n]
-            if r:
-                d, ts = r
-                for t in ts:
-                    used.add((t.coef, d if t.coef in ("PA", "WP", "QC", "WQ") else None))
-        need = lambda c: any(u[0] == c for u in used)  # noqa: E731
+        used = _vrr_factors(v, nodes)
         for i in range(len(tg)):
             E(f"R c{i} = R(0);", ind)
         E("for (int kc = 0; kc < k_cd; ++kc) {", ind)
         E("const double* __restrict__ q_ = kp + 8 * kc;", ind + 1)
-        E("const double Qx = q_[0], Qy = q_[1], Qz = q_[2], q = q_[6], Uq = q_[7];", ind + 1)
-        for d in range(3):
-            if ("QC", d) in used:
-                E(f"const R QC{AX[d]} = R(q_[{3 + d}]);", ind + 1)
-        if need("i2q") or need("i2q_r"):
-            E("const double iq = 1.0 / q;", ind + 1)
+        _emit_ket_prim(E, used, ind + 1)
         E("for (int kb = 0; kb < k_ab; ++kb) {", ind + 1)
         i2 = ind + 2
         E("const double* __restrict__ p_ = bp + FJ_SREC * kb;", i2)
-        E("const double PQx = p_[0] - Qx, PQy = p_[1] - Qy, PQz = p_[2] - Qz;", i2)
-        E("const double p = p_[6];", i2)
-        E("const double ippq = 1.0 / (p + q);", i2)
-        E("const double rho = p * q * ippq;", i2)
-        E("const double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);", i2)
-        E(f"double Fm[{L + 1}];", i2)
-        E(f"fj_boys_lds<{L}>(T, Fm, tb);" if W else f"fj_boys<{L}>(T, Fm);", i2)
-        E("const double S = p_[7] * Uq * (FJ_TWO_OVER_SQRT_PI * sqrt(rho));", i2)
-        for d in range(3):
-            if ("PA", d) in used:
-                E(f"const R PA{AX[d]} = R(p_[{3 + d}]);", i2)
-            if ("WP", d) in used:
-                E(f"const R WP{AX[d]} = R(-q * ippq * PQ{AX[d]});", i2)
-            if ("WQ", d) in used:
-                E(f"const R WQ{AX[d]} = R(p * ippq * PQ{AX[d]});", i2)
-        if need("i2p"):
-            E("const R i2p = R(0.5 * p_[8]);", i2)
-        if need("i2p_r"):
-            E("const R i2p_r = R(0.5 * p_[8] * rho * p_[8]);", i2)
-        if need("i2q"):
-            E("const R i2q = R(0.5 * iq);", i2)
-        if need("i2q_r"):
-            E("const R i2q_r = R(0.5 * iq * rho * iq);", i2)
-        if need("i2pq"):
-            E("const R i2pq = R(0.5 * ippq);", i2)
-        for n in v.order:
-            if n not in nodes:
-                continue
-            r = v.terms[n]
-            if not r:
-                E(f"const R {_vname(n)} = R(S * Fm[{n[2]}]);", i2)
-                continue
-            d, ts = r
-            parts = []
-            for t in ts:
-                c = t.coef
-                ch = _vname(t.child)
-                if c in ("PA", "WP", "QC", "WQ"):
-                    parts.append(f"{c}{AX[d]} * {ch}")
-                else:
-                    m = t.mult
-                    sign = "-" if m < 0 else "+"
-                    f = c if abs(m) == 1 else f"(R({abs(m)}) * {c})"
-                    parts.append(f"{sign} {f} * {ch}")
-            expr = parts[0]
-            for q_ in parts[1:]:
-                expr += (" " + q_) if q_[0] in "+-" else (" + " + q_)
-            E(f"const R {_vname(n)} = {expr};", i2)
+        _emit_prim_vrr(E, v, L, nodes, used,
+                       f"fj_boys_lds<{L}>(T, Fm, tb);" if W else f"fj_boys<{L}>(T, Fm);", i2)
         for i, (e, f) in enumerate(tg):
             E(f"c{i} += {_vname((e, f, 0))};", i2)
         E("}", ind + 1)
@@ -1525,3 +1484,380 @@ def emit_quartet_staged(cls, split: bool = False) -> str:
             E("}")
     E("}", 0)
     return E.text()
+
+# ---------------------------------------------------------------------------
+# The quartet-cooperative form (csrc/fj_coop.h) of a class through d: a
+# wavefront per bra pair and up to NQ kets, lanes over their primitive
+# quartets, boundaries summed in LDS, HRR and digestion once per quartet.
+
+COOP_LDS = 159 * 1024   # of a CU's 160 KB
+COOP_NQ_MAX = 32
+
+
+def coop_tune(cls) -> tuple[int, int, int, int]:
+    """(live values per VRR group, workgroups per CU, targets summed over the
+    lanes at a time, doubles of a wavefront's X and density blocks). The VRR
+    is a long dependent chain, so a second wavefront per SIMD to switch to is
+    worth more than large groups, until the groups get so small that they
+    recompute and spill too much. Measured on the 40-atom s,s,p,d cluster,
+    every launch alone: with the per-lane form's 220 live and one wavefront
+    per SIMD the launches sum to 88 ms, with 100 live and two 78 ms, with 60
+    live and three 147 ms (four wavefronts per quartet; the per-lane form
+    itself 102 ms), and with a wavefront per quartet and the choices below 67
+    ms. By class:
+    * at most 18 targets: four workgroups fit ((ss|ds) 1.29 -> 1.11 ms,
+      (ss|ss) 0.79 -> 0.57 ms);
+    * (dd|dd), (pd|dd), (dp|dd) and (pd|pd): one workgroup per CU with
+      large groups ((dd|dd) 9.9 ms against 15.1, (pd|dd) 7.7 against 8.3,
+      (dp|dd) 3.4 against 3.7, (pd|pd) 1.7 against 2.1);
+    * (sd|dd), (ds|dd), (pd|dp): less scratch, so more quartets per wavefront
+      ((pd|dp) 1.72 -> 1.49 ms);
+    * five classes of 54 to 114 targets spill in their groups at 100 live
+      and gain by those at 84 ((sd|sd) 1.49 -> 1.16 ms, (pd|ds) 2.63 -> 2.27
+      ms); the others lose by them ((sd|pd) 2.60 -> 3.13 ms)."""
+    c = tuple(cls)
+    if len(vrr_dag(c).targets) <= 18:
+        return 60, 4, 8, 600
+    if c == (2, 2, 2, 2):
+        return 220, 1, 16, 1600
+    if c in {(1, 2, 2, 2), (2, 1, 2, 2), (1, 2, 1, 2)}:
+        return 220, 1, 16, 1100
+    if c in {(0, 2, 2, 2), (2, 0, 2, 2), (1, 2, 2, 1)}:
+        return 100, 2, 8, 900
+    small = {(0, 2, 2, 0), (0, 2, 1, 1), (0, 2, 0, 2), (1, 1, 2, 0), (1, 2, 2, 0)}
+    return (84 if c in small else 100), 2, 16, 1100
+
+
+def coop_shape(cls) -> dict:
+    """The class's sizes in the cooperative kernel: components, the doubles
+    of a quartet's boundary (half-transformed in place), X's row stride, the
+    F elements, the quartets of a pass through phases B to D (QW), the a
+    components of an X slice (SA) and the quartets of a wavefront (NQ)."""
+    la, lb, lc, ld = cls
+    na, nb, nc, nd = (n_cart(x) for x in cls)
+    ne = sum(n_cart(n) for n in range(la, la + lb + 1))
+    nf = sum(n_cart(n) for n in range(lc, lc + ld + 1))
+    reg = max(ne, na * nb) * nf
+    xs = (nc * nd) | 1
+    no = na * nb + nc * nd + (na + nb) * (nc + nd)
+    live, wgs, chunk, x = coop_tune(cls)
+    qw = max(1, min(8, x // (na * nb * xs + no)))
+    sa = na if qw > 1 else max(1, min(na, (x - no) // (nb * xs)))
+    wt = max(chunk * 65, qw * (sa * nb * xs + no))
+    fixed = 8 * (MAX_PRIM_PAIRS * 9 + 4 * wt + na * nb)
+    nq = (COOP_LDS // wgs - fixed) // (4 * (8 * reg + 32))
+    nq = int(max(1, min(COOP_NQ_MAX // 4, nq)))
+    qw = min(qw, nq)
+    return dict(na=na, nb=nb, nc=nc, nd=nd, ne=ne, nf=nf, reg=reg, xs=xs, no=no, qw=qw, sa=sa, wt=wt,
+                nq=nq, live=live, wgs=wgs, chunk=chunk)
+
+
+def emit_coop(cls) -> str:
+    """c_<cls>.h: the cooperative kernel's body and kernels fj_c_<cls>_k (one
+    tier) and fj_c_<cls>_km (each item in its tier)."""
+    from .hgp import closure, e_groups
+    la, lb, lc, ld = cls
+    L = sum(cls)
+    v = vrr_dag(tuple(cls))
+    name = cls_name(cls)
+    h = coop_shape(cls)
+    na, nb, nc, nd, NE, NF = (h[k] for k in ("na", "nb", "nc", "nd", "ne", "nf"))
+    NAB, REG, XS, NO, QW, SA, NQ, WT = na * nb, h["reg"], h["xs"], h["no"], h["qw"], h["sa"], h["nq"], h["wt"]
+    CH = h["chunk"]
+    eR = [e for n in range(la, la + lb + 1) for e in cartesians(n)]
+    fR = [f for n in range(lc, lc + ld + 1) for f in cartesians(n)]
+    groups = e_groups(tuple(cls), h["live"])
+    E = _Emit()
+    E(f"// generated by felizjueves_amd/gen_hip.py -- cooperative F kernel of ({la}{lb}|{lc}{ld}): "
+      f"{len(groups)} VRR groups, {len(v.targets)} boundary values", 0)
+    E('#pragma once\n#include "../fj_device.h"\n#include "../fj_coop.h"\n', 0)
+    # A: the boundary values of the lane's primitive quartets r, r + m, ... of
+    # a quartet of n (its ket primitives from kp, the bra's kab in bp),
+    # summed over the quartet's lanes into bnd[q][e][f]
+    E("template <typename R>", 0)
+    E(f"__device__ __forceinline__ void fj_ca_{name}(const double* __restrict__ bp, int kab,", 0)
+    E("const double* __restrict__ kp, int r, int m, int n, double* __restrict__ red, int lane,", 1)
+    E("unsigned mask, int q0, int nq, double* __restrict__ bnd) {", 1)
+    E("const int kc0 = r / kab, kb0 = r - kc0 * kab, mc = m / kab, mb = m - mc * kab;")
+    for gi, g in enumerate(groups):
+        tg = [(e, f) for e in eR if e in g for f in fR]
+        assert set(tg) == {(e, f) for e, f in v.targets if e in g}
+        pos = [eR.index(e) * NF + fR.index(f) for e, f in tg]
+        assert pos == list(range(pos[0], pos[0] + len(pos))), (cls, gi)
+        nodes = closure(v, [(e, f, 0) for e, f in tg])
+        used = _vrr_factors(v, nodes)
+        E(f"{{   // group {gi}")
+        for i in range(len(tg)):
+            E(f"R c{i} = R(0);", 2)
+        E("int kc = kc0, kb = kb0;", 2)
+        E("#pragma unroll 1", 0)
+        E("for (int i = r; i < n; i += m) {", 2)
+        E("const double* __restrict__ q_ = kp + 8 * kc;", 3)
+        _emit_ket_prim(E, used, 3)
+        E("const double* __restrict__ p_ = bp + FJ_SREC * kb;", 3)
+        _emit_prim_vrr(E, v, L, nodes, used, f"fj_boys<{L}>(T, Fm);", 3)
+        for i, (e, f) in enumerate(tg):
+            E(f"c{i} += {_vname((e, f, 0))};", 3)
+        E("kc += mc;", 3)
+        E("kb += mb;", 3)
+        E("if (kb >= kab) { kb -= kab; ++kc; }", 3)
+        E("}", 2)
+        for t0 in range(0, len(tg), CH):
+            cnt = min(CH, len(tg) - t0)
+            for i in range(cnt):
+                E(f"red[{i} * FJ_COOP_ROW + lane] = double(c{t0 + i});", 2)
+            E("fj_wave_sync();", 2)
+            E(f"fj_coop_reduce<{cnt}, {CH}>(red, lane, mask, q0, nq, bnd, {REG}, {pos[t0]});", 2)
+            E("fj_wave_sync();", 2)
+        E("}")
+    E("}\n", 0)
+    # B: the bra HRR of column f of one quartet's boundary w [e][f], in place [ab][f]
+    if lb:
+        E(f"__device__ __forceinline__ void fj_cb_{name}(double* __restrict__ w, double ABx, double ABy, double ABz) {{", 0)
+        _emit_side_hrr(E, la, lb, "AB", lambda i: f"w[{i * NF}]", lambda j, nm: E(f"w[{j * NF}] = {nm};"), 1)
+        E("}\n", 0)
+    # C: the ket HRR of row ab, m [f] -> X [cd]
+    E(f"__device__ __forceinline__ void fj_cc_{name}(const double* __restrict__ m, double* __restrict__ X,", 0)
+    E("double CDx, double CDy, double CDz) {", 1)
+    _emit_side_hrr(E, lc, ld, "CD", lambda i: f"m[{i}]", lambda j, nm: E(f"X[{j}] = {nm};"), 1)
+    E("}\n", 0)
+    ab = "a.bra.sep[3 * bra], a.bra.sep[3 * bra + 1], a.bra.sep[3 * bra + 2]" if lb else ""
+    cd = ("a.ket.sep[3 * K.k[q]], a.ket.sep[3 * K.k[q] + 1], a.ket.sep[3 * K.k[q] + 2]" if ld else "0.0, 0.0, 0.0")
+    phase_b = f"""
+            for (int t = lane; t < nw * {NF}; t += 64) {{
+                const int q = t / {NF};
+                fj_cb_{name}(bnd + (qs + q) * {REG} + (t - q * {NF}), {ab});
+            }}
+            fj_wave_sync();""" if lb else ""
+    # D: element o of quartet q gets x
+    store = """if (s0 == 0 && s1 == 1) {
+                    unsafeAtomicAdd(fab + i * %d + j, x);
+                } else {
+                    const int oc = a.ket.ao[2 * k], od = a.ket.ao[2 * k + 1];
+                    const int ro = s0 == 0 ? oa : s0 == 1 ? ob : oc, co = s1 == 2 ? oc : od;
+                    unsafeAtomicAdd(S.F + (size_t)(ro + i) * n_ao + co + j, x);
+                }""" % nb
+    # whether any of quartet q's primitives are this part's
+    here = "K.lane0[q] < (part + 1) * 64 && K.lane0[q] + K.lanes[q] > part * 64"
+    if SA == na:
+        phase_cd = f"""            for (int t = lane; t < nw * {NAB}; t += 64) {{
+                const int q = qs + t / {NAB}, ab = t % {NAB};
+                fj_cc_{name}(bnd + q * {REG} + ab * {NF}, X + t * {XS}, {cd});
+            }}
+            fj_wave_sync();
+            for (int t = lane; t < nw * {NO}; t += 64) {{
+                const int u = t / {NO}, q = qs + u, k = K.k[q];
+                if (!({here})) continue;
+                int s0, s1, i, j;
+                B::of(t % {NO}, s0, s1, i, j);
+                const double x = B::template sum<{XS}>(X + u * {NAB * XS}, wd + u * {NO}, s0, s1, i, j, 0, {na});
+                {store}
+            }}
+"""
+    else:
+        nacc = -(-NO // 64)
+        phase_cd = f"""            const int q = qs, k = K.k[q];   // one quartet per pass
+            double acc[{nacc}] = {{}};
+            for (int a0 = 0; a0 < {na}; a0 += {SA}) {{
+                const int a1 = min(a0 + {SA}, {na});
+                for (int t = lane; t < (a1 - a0) * {nb}; t += 64)
+                    fj_cc_{name}(bnd + q * {REG} + (a0 * {nb} + t) * {NF}, X + t * {XS}, {cd});
+                fj_wave_sync();
+#pragma unroll
+                for (int u = 0; u < {nacc}; ++u) {{
+                    if (lane + 64 * u >= {NO}) continue;
+                    int s0, s1, i, j;
+                    B::of(lane + 64 * u, s0, s1, i, j);
+                    acc[u] += B::template sum<{XS}>(X, wd, s0, s1, i, j, a0, a1);
+                }}
+                fj_wave_sync();
+            }}
+#pragma unroll
+            for (int u = 0; u < {nacc}; ++u) {{
+                if (lane + 64 * u >= {NO} || !({here})) continue;
+                const double x = acc[u];
+                int s0, s1, i, j;
+                B::of(lane + 64 * u, s0, s1, i, j);
+                {store}
+            }}
+"""
+    E.lines.append(f"""// One work item (a bra pair and its list of kets), part `part` of `parts`
+// workgroups sharing its primitive quartets. MIXED: in the FP32 tier when f32.
+template <bool MIXED>
+__device__ __forceinline__ void fj_citem_{name}(const FjFArgs& a, int it, bool f32, int part, int parts,
+                                             double* __restrict__ bsh, double* __restrict__ bnd_,
+                                             double* __restrict__ wt, double* __restrict__ fab,
+                                             FjCoopKets<{NQ}>* __restrict__ K_) {{
+    typedef FjCoopBlocks<{na}, {nb}, {nc}, {nd}> B;
+    static_assert(B::N == {NO}, "elements of the F blocks");
+    const int4 w = a.work[it];
+    const int bra = w.x, kb_lo = (w.z >> 16) & 0xff, kb_n = (w.z >> 24) & 0xff;
+    const FjSys S = a.sys[w.z & 0xffff];
+    int kb0, kab;
+    fj_side_range(a.bra, bra, kb0, kab);
+    if (kab > FJ_MAX_PRIM_PAIRS || kb_lo >= kab) return;   // uniform; the host emits neither
+    kb0 += kb_lo;
+    kab = kb_n ? min(kab - kb_lo, kb_n) : kab - kb_lo;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int i = tid; i < kab; i += FJ_COOP_THREADS) {{
+        const double* __restrict__ r = a.bra.prim + 8 * (size_t)(kb0 + i);
+        double* s = bsh + FJ_SREC * i;
+#pragma unroll
+        for (int f = 0; f < 8; ++f) s[f] = r[f];
+        s[8] = 1.0 / r[6];
+    }}
+    for (int i = tid; i < {NAB}; i += FJ_COOP_THREADS) fab[i] = 0.0;
+    __syncthreads();
+    const int n_ao = S.n_ao, sa = a.bra.sh[2 * bra], sb = a.bra.sh[2 * bra + 1];
+    const int oa = a.bra.ao[2 * bra], ob = a.bra.ao[2 * bra + 1];
+    // this wavefront's scratch, boundaries and kets: every fourth one, or,
+    // where the item has fewer than four, a quarter of the primitives of all
+    double* const wv = wt + wave * {WT};
+    double* const bnd = bnd_ + wave * {NQ * REG};
+    FjCoopKets<{NQ}>& K = K_[wave];
+    const int step = w.w - w.y < FJ_COOP_WAVES ? 1 : FJ_COOP_WAVES;
+    if (step == 1) {{
+        part = part * FJ_COOP_WAVES + wave;
+        parts *= FJ_COOP_WAVES;
+    }}
+    for (int first = w.y + (step == 1 ? 0 : wave); first < w.w; first += step * {NQ}) {{
+        const int nq = fj_coop_kets<{NQ}>(a, S, K, bra, kab, first, step,
+                                          min({NQ}, (w.w - first + step - 1) / step), parts);
+        if (nq == 0 || K.lane0[nq - 1] + K.lanes[nq - 1] <= part * 64) continue;   // uniform over the wavefront
+        for (int i = lane; i < nq * {REG}; i += 64) bnd[i] = 0.0;
+        fj_wave_sync();
+        // the lane's quartet, and the quartets of its run of {CH} lanes
+        const int g = part * 64 + lane, gr = part * 64 + (lane & ~{CH - 1});
+        int mine = -1, q0 = 0;
+        unsigned mask = 0;
+        for (int q = 0; q < nq; ++q) {{
+            const int l0 = K.lane0[q], l1 = l0 + K.lanes[q];
+            if (g >= l0 && g < l1) mine = q;
+            if (l1 <= gr) q0 = q + 1;
+            else if (l1 < gr + {CH}) mask |= 1u << (l1 - 1 - gr);
+        }}
+        {{
+            const int q = mine < 0 ? 0 : mine;
+            const bool any = mine >= 0;
+            const int n = any ? K.n[q] : 0, m = any ? K.lanes[q] : 1, r = any ? g - K.lane0[q] : 0;
+            const double* __restrict__ kp = a.ket.prim + 8 * (size_t)(any ? K.p0[q] : 0);
+            if (MIXED && f32)
+                fj_ca_{name}<float>(bsh, kab, kp, r, m, n, wv, lane, mask, q0, nq, bnd);
+            else
+                fj_ca_{name}<double>(bsh, kab, kp, r, m, n, wv, lane, mask, q0, nq, bnd);
+        }}
+        for (int qs = 0; qs < nq; qs += {QW}) {{
+            const int nw = min({QW}, nq - qs);{phase_b}
+            // the weighted density blocks of the pass's quartets
+            double* const X = wv;
+            double* const wd = wv + {QW} * {SA * nb * XS};
+            for (int t = lane; t < nw * {NO}; t += 64) {{
+                const int q = qs + t / {NO}, k = K.k[q];
+                int s0, s1, i, j;
+                B::of(t % {NO}, s0, s1, i, j);
+                const int oc = a.ket.ao[2 * k], od = a.ket.ao[2 * k + 1];
+                double deg = 1.0;
+                if (sa == sb) deg *= 0.5;
+                if (a.ket.sh[2 * k] == a.ket.sh[2 * k + 1]) deg *= 0.5;
+                if (a.diag && k == bra) deg *= 0.5;
+                const int ro = s0 == 0 ? oa : s0 == 1 ? ob : oc, co = s1 == 1 ? ob : s1 == 2 ? oc : od;
+                const bool coul = (s0 == 0 && s1 == 1) || s0 == 2;
+                wd[t] = (coul ? 2.0 * deg : -0.5 * deg) * S.D[(size_t)(ro + i) * n_ao + co + j];
+            }}
+{phase_cd}            fj_wave_sync();
+        }}
+    }}
+    __syncthreads();
+    for (int i = tid; i < {NAB}; i += FJ_COOP_THREADS) {{
+        const double s = fab[i];
+        if (s != 0.0) unsafeAtomicAdd(S.F + (size_t)(oa + i / {nb}) * n_ao + ob + i % {nb}, s);
+    }}
+}}
+
+template <bool MIXED>
+__global__ void __launch_bounds__(FJ_COOP_THREADS, {h["wgs"]}) fj_c_{name}_k(FjFArgs a, const int* parent) {{
+    __shared__ double bsh[FJ_MAX_PRIM_PAIRS * FJ_SREC], bnd[{4 * NQ * REG}], wt[{4 * WT}], fab[{NAB}];
+    __shared__ FjCoopKets<{NQ}> K[FJ_COOP_WAVES];
+    const int it = (int)blockIdx.x;
+    fj_citem_{name}<MIXED>(a, it, MIXED && !fj_item_fp64(a, parent[it]), (int)blockIdx.y, (int)gridDim.y, bsh, bnd, wt,
+                        fab, K);
+}}
+""")
+    return E.text()
+
+
+def coop_entry(cls) -> str:
+    """fj_fc_<cls>, the cooperative launch of a builder work list."""
+    n = cls_name(cls)
+    return (f"int fj_claunch_{n}_mx(hipStream_t s, dim3 grid, const FjFArgs& a, const int* parent);\n\n"
+            f'extern "C" int fj_fc_{n}(hipStream_t s, int parts, const FjSide* bra, const FjSide* ket,\n'
+            "                        const int* work, int n_work, const int* ket_list, const int* parent,\n"
+            "                        const int* tier, const FjSys* sys, int diag, double tau) {\n"
+            "    if (!bra || !ket || !work || !sys || !ket_list || (tier && !parent)) return FJ_ERR_ARG;\n"
+            "    if (parts < 1 || parts > 64) return FJ_ERR_ARG;\n"
+            "    if (n_work <= 0 || ket->n <= 0) return 0;\n"
+            "    FjFArgs a;\n"
+            "    a.bra = *bra; a.ket = *ket;\n"
+            "    a.work = reinterpret_cast<const int4*>(work);\n"
+            "    a.ket_list = ket_list; a.sys = sys;\n"
+            "    a.one = FjSys{nullptr, nullptr, nullptr, 0, 0};\n"
+            "    a.diag = diag; a.tau = tau;\n"
+            "    a.ws = nullptr; a.ws_doubles = 0; a.n_bx = n_work; a.n_items = n_work;\n"
+            "    a.n_fp64 = 0; a.tier = tier;\n"
+            "    const dim3 grid((unsigned)n_work, (unsigned)parts);\n"
+            f"    if (tier) return fj_claunch_{n}_mx(s, grid, a, parent);\n"
+            f"    hipLaunchKernelGGL(fj_c_{n}_k<false>, grid, dim3(FJ_COOP_THREADS), 0, s, a, parent);\n"
+            "    return (int)hipGetLastError();\n}\n")
+
+
+def generate_coop(classes, out: Path = GEN) -> list[Path]:
+    """c_<cls>.h, c_<cls>.hip (the FP64 kernel and the entry) and c_<cls>_mx.hip
+    (the mixed-tier kernel) of every class."""
+    out.mkdir(parents=True, exist_ok=True)
+    files = []
+    for cls in classes:
+        n = cls_name(cls)
+        gen = "// generated by felizjueves_amd/gen_hip.py -- cooperative F kernel\n"
+        texts = {f"c_{n}.h": emit_coop(cls),
+                 f"c_{n}.hip": gen + f'#include "c_{n}.h"\n\n' + coop_entry(cls),
+                 f"c_{n}_mx.hip": gen + f'#include "c_{n}.h"\n\n'
+                 f"int fj_claunch_{n}_mx(hipStream_t s, dim3 grid, const FjFArgs& a, const int* parent) {{\n"
+                 f"    hipLaunchKernelGGL(fj_c_{n}_k<true>, grid, dim3(FJ_COOP_THREADS), 0, s, a, parent);\n"
+                 f"    return (int)hipGetLastError();\n}}\n"}
+        for fname, text in texts.items():
+            p = out / fname
+            if not p.exists() or p.read_text() != text:
+                p.write_text(text)
+        files += [out / f"c_{n}.hip", out / f"c_{n}_mx.hip"]
+    # the kets a workgroup takes at once, for the host's work lists
+    p = out / "fj_coop_table.hip"
+    L = ["// generated by felizjueves_amd/gen_hip.py -- kets per batch of the cooperative kernels",
+         '#include "../fj_device.h"', "",
+         'extern "C" int fj_fc_batch(int la, int lb, int lc, int ld) {',
+         "    if (la < 0 || lb < 0 || lc < 0 || ld < 0 || la > 3 || lb > 3 || lc > 3 || ld > 3) return 0;",
+         "    switch (((la * 4 + lb) * 4 + lc) * 4 + ld) {"]
+    for cls in classes:
+        la, lb, lc, ld = cls
+        L.append(f"        case {((la * 4 + lb) * 4 + lc) * 4 + ld}: return {4 * coop_shape(cls)['nq']};")
+    L += ["        default: return 0;   // no cooperative kernel", "    }", "}", ""]
+    text = "\n".join(L)
+    if not p.exists() or p.read_text() != text:
+        p.write_text(text)
+    return files + [p]
+
+
+COOP_BEGIN, COOP_END = ("/* BEGIN COOPERATIVE CLASSES (written by felizjueves_amd/gen_hip.py) */",
+                        "/* END COOPERATIVE CLASSES */")
+
+
+def write_coop_header(classes) -> None:
+    """The cooperative entries' section of include/fj_mi355x.h."""
+    decl = "\n".join(
+        f"int fj_fc_{cls_name(c)}(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,\n"
+        f"    const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,\n"
+        f"    const FjSys* sys, int diag, double tau);" for c in classes) + "\n"
+    cur = HEADER.read_text()
+    i, j = cur.index(COOP_BEGIN), cur.index(COOP_END)
+    text = cur[:i + len(COOP_BEGIN)] + "\n" + decl + cur[j:]
+    if text != cur:
+        HEADER.write_text(text)

@@ -158,6 +158,26 @@ def call_fxm(cls, threads: int, bra: FjSide, ket: FjSide, work, n_work: int, n_f
     check(rc, fn.__name__)
 
 
+def coop_batch(cls) -> int:
+    """The kets a workgroup of fj_fc_<cls> takes at once (0: no such form)."""
+    fn = lib().fj_fc_batch
+    fn.restype = C.c_int
+    return int(fn(*[C.c_int(x) for x in cls]))
+
+
+def call_fc(cls, parts: int, bra: FjSide, ket: FjSide, work, n_work: int, ket_list, parent, tier, sys,
+            diag: int, tau: float, stream=None) -> None:
+    """One quartet-cooperative launch fj_fc_<cls>: `work`, `ket_list` as for
+    call_fx, each item over `parts` workgroups; with `tier` (a device int32
+    array) item i in tier[parent[i]], else in FP64."""
+    fn = getattr(lib(), "fj_fc_" + "".join(map(str, cls)))
+    fn.restype = C.c_int
+    rc = fn(C.c_void_p(stream_handle(stream)), C.c_int(parts), C.byref(bra), C.byref(ket),
+            C.c_void_p(ptr(work)), C.c_int(n_work), C.c_void_p(ptr(ket_list)), C.c_void_p(ptr(parent)),
+            C.c_void_p(ptr(tier)), C.c_void_p(ptr(sys)), C.c_int(diag), C.c_double(tau))
+    check(rc, fn.__name__)
+
+
 class FjTierSel(C.Structure):
     """Mirror of ``FjTierSel`` in include/fj_mi355x.h (device pointers)."""
 

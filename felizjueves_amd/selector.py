@@ -14,7 +14,7 @@ import numpy as np
 
 from . import native
 from .features import N_FEATURES, tile_features
-from .fock import FP32, FP64, FockBuilder
+from .fock import FP32, FP64, WS_MAX_BYTES, FockBuilder
 
 def item_features(fb: FockBuilder, L, w) -> np.ndarray:
     """The tile features (features.tile_features) of work item
@@ -41,6 +41,9 @@ def probe_errors(fb: FockBuilder, D: np.ndarray, max_items: int = 4096, seed: in
         sel = rng.choice(len(items), size=max_items, replace=False)
         items = [items[i] for i in sorted(sel)]
     feats, errs, des = [], [], []
+    # the per-lane form in both tiers, whatever form the builder's launches take
+    need = max([native.workspace_bytes(L.cls, L.threads, L.work.shape[0]) for L in fb.launches] + [8])
+    ws = torch.empty(min(WS_MAX_BYTES, need) // 8, dtype=torch.float64, device=Dd.device)
     native.density_blocks(fb.shell_ao[0], fb.shell_size[0], Dd, fb.Dsh)
     batch = 512
     for s0 in range(0, len(items), batch):
@@ -59,7 +62,7 @@ def probe_errors(fb: FockBuilder, D: np.ndarray, max_items: int = 4096, seed: in
                 w[:, 2] = (w[:, 2] & ~0xffff) | np.array([j for j, _ in lst], dtype=np.int32)
                 wd = native.to_dev(w)
                 native.call_fx(L.cls, L.threads, tier, L.bra.side, L.ket.side, wd, w.shape[0],
-                               sys, L.diag, fb.tau, None, L.ket_list_dev, fb._workspace(0))
+                               sys, L.diag, fb.tau, None, fb.per_lane(L)[1], ws)
         torch.cuda.synchronize()
         d = (F[FP32] - F[FP64])
         d = d + d.transpose(1, 2)

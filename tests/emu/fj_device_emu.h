@@ -17,7 +17,7 @@ using std::min; using std::max; using std::fma; using std::sqrt; using std::exp;
 #define __host__
 #define __forceinline__ inline
 #define __noinline__ __attribute__((noinline))
-#define __launch_bounds__(x)
+#define __launch_bounds__(...)
 #define __shared__ static
 #define __restrict__ __restrict
 struct dim3 { unsigned x, y, z; dim3(unsigned a = 1, unsigned b = 1, unsigned c = 1) : x(a), y(b), z(c) {} };
@@ -84,6 +84,8 @@ inline fj_v4d fj_mfma_f64_16x16x4(double a, double b, fj_v4d c) {
     }
     return c;
 }
+// the lanes of a wavefront meet at its barrier (g_wbar, set by the driver)
+inline void fj_wave_sync() { g_wbar[threadIdx.x >> 6]->arrive_and_wait(); }
 inline void unsafeAtomicAdd(double* p, double v) { std::atomic_ref<double>(*p).fetch_add(v); }
 inline double atomicAdd(double* p, double v) { return std::atomic_ref<double>(*p).fetch_add(v); }
 inline void fj_side_range(const FjSide& s, int i, int& k0, int& k) {
