@@ -63,6 +63,7 @@ def sources(lmax: int = LMAX) -> list[Path]:
     files += split
     files.append(gen_hip.write_df())   # density fitting: metric and three-center entries
     files.append(gen_hip.write_gf())   # the fused two-electron gradient's entries
+    files += gen_hip.generate_gfquad()
     mmd = gen_mmd.generate(MMD_LMAX, k_lmax=MMD_K_LMAX)
     gen_mmd.write_header(MMD_LMAX, MMD_K_LMAX)
     return [CSRC / "fj_runtime.hip", CSRC / "fj_mlp.hip", CSRC / "fj_plan.hip", CSRC / "fj_kloop.hip",
@@ -79,10 +80,12 @@ def _compile(src: Path, extra: list[str], force: bool = False) -> tuple[Path, fl
         deps.append(hdr)
     if src.name.startswith("c_"):
         deps.append(CSRC / "fj_coop.h")
+    if src.name.startswith("gq_"):
+        deps += [CSRC / "fj_kloop.h", CSRC / "fj_gfloop.h", CSRC / "fj_gfquad.h"]
     if src.name in ("fj_kloop.hip", "fj_dfloop.hip", "fj_gfloop.hip"):
         deps.append(CSRC / "fj_kloop.h")
     if src.name == "fj_gfloop.hip":
-        deps.append(CSRC / "fj_gfloop.h")
+        deps += [CSRC / "fj_gfloop.h", CSRC / "gen" / "gq_table.h"]
     if src.name == "fj_dfloop.hip":
         deps.append(CSRC / "fj_dfloop.h")
     if src.name == "fj_kloop.hip":

@@ -41,6 +41,9 @@
 // No screen (kernel_gf.py:82-85: the F screen bounds an integral, not its
 // derivative): every unique quartet of a launch is visited.
 //
+// Launches of 256 lanes, the default, run fj_gfquad.h instead, on the matrix
+// cores; this form takes any width of whole wavefronts.
+//
 // The includer provides fj_device.h (the device one, or the CPU emulation);
 // the launcher and the per-class entries are in fj_gfloop.hip.
 #pragma once
@@ -192,6 +195,69 @@ __device__ __forceinline__ void fj_gf_tile(const double* __restrict__ A, int sam
     }
 }
 
+// Work item q0 of a launch: with a job table, g becomes the item's job; the
+// item's quartet (bra, ket) and primitive quartets pq0 .. pq1 - 1, and the
+// quartet's degeneracy 1/|Stab| (kernel_gf.py:591-606: 1/2 for a = b, for
+// c = d, and for the pair met with itself on the diagonal launch).
+__device__ __forceinline__ double fj_gf_item(FjGfArgs& g, const FjGfJob* jobs, int n_jobs, long long q0,
+                                             int& pq0, int& pq1, int& bra, int& ket) {
+    const FjGfArgs g0 = g;
+    long long q = q0;
+    if (jobs) {
+        int lo = 0, hi = n_jobs - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (jobs[mid].q0 <= q0) lo = mid;
+            else hi = mid - 1;
+        }
+        const FjGfJob J = jobs[lo];
+        q = q0 - J.q0;
+        g.n_bra = J.n_bra;
+        g.n_ket = J.n_ket;
+        g.k_ab = J.k_ab;
+        g.k_cd = J.k_cd;
+        g.diag = J.diag;
+        g.chunk = J.chunk;
+        g.bra_prim = g0.bra_prim + J.bra_prim;
+        g.ket_prim = g0.bra_prim + J.ket_prim;
+        g.AB = g0.AB + 3 * (size_t)J.bra_row;
+        g.CD = g0.AB + 3 * (size_t)J.ket_row;
+        g.bra_sh = g0.bra_sh + 2 * (size_t)J.bra_row;
+        g.ket_sh = g0.bra_sh + 2 * (size_t)J.ket_row;
+        g.bra_ao = g0.bra_ao + 2 * (size_t)J.bra_row;
+        g.ket_ao = g0.bra_ao + 2 * (size_t)J.ket_row;
+        g.bra_at = g0.bra_at + 2 * (size_t)J.bra_row;
+        g.ket_at = g0.bra_at + 2 * (size_t)J.ket_row;
+    }
+    const int n_pq = g.k_ab * g.k_cd;
+    const int n_ch = (n_pq + g.chunk - 1) / g.chunk;
+    const long long qi = q / n_ch;
+    pq0 = (int)(q - qi * n_ch) * g.chunk;
+    pq1 = pq0 + g.chunk < n_pq ? pq0 + g.chunk : n_pq;
+    q = qi;
+    // the quartet: (bra, ket), ket >= bra on the diagonal launch (its upper
+    // triangle, row-major), every pair otherwise
+    if (g.diag) {
+        const long long n = g.n_bra;
+        const double b2 = (double)(2 * n + 1);
+        long long b = (long long)((b2 - sqrt(b2 * b2 - 8.0 * (double)q)) * 0.5);
+        if (b < 0) b = 0;
+        if (b > n - 1) b = n - 1;
+        while (b > 0 && b * n - b * (b - 1) / 2 > q) --b;
+        while (b + 1 < n && (b + 1) * n - (b + 1) * b / 2 <= q) ++b;
+        bra = (int)b;
+        ket = (int)(b + (q - (b * n - b * (b - 1) / 2)));
+    } else {
+        bra = (int)(q / g.n_ket);
+        ket = (int)(q - (long long)bra * g.n_ket);
+    }
+    double deg = 1.0;
+    if (g.la == g.lb && g.bra_sh[2 * bra] == g.bra_sh[2 * bra + 1]) deg *= 0.5;
+    if (g.lc == g.ld && g.ket_sh[2 * ket] == g.ket_sh[2 * ket + 1]) deg *= 0.5;
+    if (g.diag && ket == bra) deg *= 0.5;
+    return deg;
+}
+
 }  // namespace
 
 // One workgroup's share of a launch: work items blockIdx.x, + gridDim.x,
@@ -269,65 +335,10 @@ __device__ __forceinline__ void fj_gf_body(const FjGfArgs& g0, const FjGfLds& o,
 
     for (long long q0 = (long long)blockIdx.x; q0 < n_items; q0 += (long long)gridDim.x) {
         FjGfArgs g = g0;
-        long long q = q0;
-        if (jobs) {
-            int lo = 0, hi = n_jobs - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (jobs[mid].q0 <= q0) lo = mid;
-                else hi = mid - 1;
-            }
-            const FjGfJob J = jobs[lo];
-            q = q0 - J.q0;
-            g.n_bra = J.n_bra;
-            g.n_ket = J.n_ket;
-            g.k_ab = J.k_ab;
-            g.k_cd = J.k_cd;
-            g.diag = J.diag;
-            g.chunk = J.chunk;
-            g.bra_prim = g0.bra_prim + J.bra_prim;
-            g.ket_prim = g0.bra_prim + J.ket_prim;
-            g.AB = g0.AB + 3 * (size_t)J.bra_row;
-            g.CD = g0.AB + 3 * (size_t)J.ket_row;
-            g.bra_sh = g0.bra_sh + 2 * (size_t)J.bra_row;
-            g.ket_sh = g0.bra_sh + 2 * (size_t)J.ket_row;
-            g.bra_ao = g0.bra_ao + 2 * (size_t)J.bra_row;
-            g.ket_ao = g0.bra_ao + 2 * (size_t)J.ket_row;
-            g.bra_at = g0.bra_at + 2 * (size_t)J.bra_row;
-            g.ket_at = g0.bra_at + 2 * (size_t)J.ket_row;
-        }
-        // the item: its quartet q and primitive quartets pq0 .. pq1 - 1
-        const int n_pq = g.k_ab * g.k_cd;
-        const int n_ch = (n_pq + g.chunk - 1) / g.chunk;
-        const long long qi = q / n_ch;
-        const int pq0 = (int)(q - qi * n_ch) * g.chunk;
-        const int pq1 = pq0 + g.chunk < n_pq ? pq0 + g.chunk : n_pq;
-        q = qi;
-        // the quartet: (bra, ket), ket >= bra on the diagonal launch (its
-        // upper triangle, row-major), every pair otherwise
-        int bra, ket;
-        if (g.diag) {
-            const long long n = g.n_bra;
-            const double b2 = (double)(2 * n + 1);
-            long long b = (long long)((b2 - sqrt(b2 * b2 - 8.0 * (double)q)) * 0.5);
-            if (b < 0) b = 0;
-            if (b > n - 1) b = n - 1;
-            while (b > 0 && b * n - b * (b - 1) / 2 > q) --b;
-            while (b + 1 < n && (b + 1) * n - (b + 1) * b / 2 <= q) ++b;
-            bra = (int)b;
-            ket = (int)(b + (q - (b * n - b * (b - 1) / 2)));
-        } else {
-            bra = (int)(q / g.n_ket);
-            ket = (int)(q - (long long)bra * g.n_ket);
-        }
+        int pq0, pq1, bra, ket;
+        const double deg = fj_gf_item(g, jobs, n_jobs, q0, pq0, pq1, bra, ket);
         const int oa = g.bra_ao[2 * bra], ob = g.bra_ao[2 * bra + 1];
         const int oc = g.ket_ao[2 * ket], od = g.ket_ao[2 * ket + 1];
-        // the degeneracy 1/|Stab| (kernel_gf.py:591-606): 1/2 for a = b, for
-        // c = d, and for the pair met with itself on the diagonal launch
-        double deg = 1.0;
-        if (la == lb && g.bra_sh[2 * bra] == g.bra_sh[2 * bra + 1]) deg *= 0.5;
-        if (lc == ld && g.ket_sh[2 * ket] == g.ket_sh[2 * ket + 1]) deg *= 0.5;
-        if (g.diag && ket == bra) deg *= 0.5;
 
         __syncthreads();   // the previous quartet's readers of W and red are done
         {

@@ -3,6 +3,7 @@
 // fj_gf_<la><lb><lc><ld> (gen/gf_entries.hip) call it.
 #include "fj_device.h"
 #include "fj_gfloop.h"
+#include "gen/gq_table.h"
 
 static constexpr long long GF_GRID = 8192;   // workgroups per launch, at most
 static constexpr long long GF_ITEMS = 2048;  // work items a launch aims for
@@ -18,6 +19,13 @@ static int fj_gf_chunk(long long n_q, int n_pq, int B) {
     int chunk = (int)((n_pq + pieces - 1) / pieces);
     chunk = (chunk + B - 1) / B * B;
     return chunk < n_pq ? chunk : n_pq;
+}
+
+// The kernel of a launch at `threads` lanes: at 256 (the default width) the
+// matrix-core one (fj_gfquad.h; the stream's classes), NULL for the loop form,
+// which takes any width: it alone runs narrower workgroups.
+static fj_gfquad_t fj_gf_quad(int la, int lb, int lc, int ld, int threads) {
+    return threads == 256 ? fj_gfquad_for(la, lb, lc, ld) : nullptr;
 }
 
 // One launch of class (la lb | lc ld) over packed sides (the upstream gf_
@@ -45,6 +53,15 @@ extern "C" int fj_gf_loop(hipStream_t s, int la, int lb, int lc, int ld, int thr
     if ((long long)k_ab * k_cd > 0x7fffffffLL) return FJ_ERR_DEGREE;
     const long long n_q = diag ? (long long)n_bra * (n_bra + 1) / 2 : (long long)n_bra * n_ket;
     const int n_pq = k_ab * k_cd;
+    if (fj_gfquad_t quad = fj_gf_quad(la, lb, lc, ld, threads)) {
+        // few quartets: their rows of primitives (one bra primitive each) in pieces
+        const int pieces = (int)(n_q >= GF_ITEMS ? 1 : (GF_ITEMS + n_q - 1) / n_q);
+        const int chunk = (k_ab + pieces - 1) / pieces * k_cd;
+        const FjGfArgs g{la, lb, lc, ld, n_bra, n_ket, k_ab, k_cd, n_atom, n_ao, diag, chunk, bra_prim, AB, bra_sh,
+                         bra_ao, bra_at, ket_prim, CD, ket_sh, ket_ao, ket_at, D, G};
+        const long long n_items = n_q * ((n_pq + chunk - 1) / chunk);
+        return quad(s, (unsigned)(n_items < GF_GRID ? n_items : GF_GRID), &g, nullptr, 0, n_items);
+    }
     const FjGfLds o = fj_gf_plan(la, lb, lc, ld, n_pq, threads);
     // a launch of few quartets splits each quartet's primitive quartets over
     // several workgroups, so that about GF_ITEMS work items fill the chip
@@ -89,10 +106,12 @@ extern "C" int fj_gf_jobs(hipStream_t s, int la, int lb, int lc, int ld, int thr
     if (n_jobs == 0 || n_items == 0) return 0;
     if (max_pq < 1) return FJ_ERR_DEGREE;
     if (!jobs || !prim || !sep || !sh || !ao || !at || !D || !G) return FJ_ERR_ARG;
-    const FjGfLds o = fj_gf_plan(la, lb, lc, ld, max_pq, threads);
     FjGfArgs g{la, lb, lc, ld, 0, 0, 0, 0, n_atom, n_ao, 0, 1, prim, sep, sh, ao, at,
                prim, sep, sh, ao, at, D, G};
     const long long grid = n_items < GF_GRID ? n_items : GF_GRID;
+    if (fj_gfquad_t quad = fj_gf_quad(la, lb, lc, ld, threads))
+        return quad(s, (unsigned)grid, &g, jobs, n_jobs, n_items);
+    const FjGfLds o = fj_gf_plan(la, lb, lc, ld, max_pq, threads);
     hipLaunchKernelGGL(fj_gfjobs_k, dim3((unsigned)grid), dim3(threads), (size_t)o.bytes, s, g, o, jobs,
                        n_jobs, n_items);
     return (int)hipGetLastError();

@@ -890,6 +890,38 @@ def emit_gf_entries() -> str:
     return "\n".join(L)
 
 
+def generate_gfquad(out: Path = GEN) -> list[Path]:
+    """gq_<cls>.hip, the matrix-core gradient kernel's launch of one class
+    each, and gq_table.h, their dispatch."""
+    out.mkdir(parents=True, exist_ok=True)
+    sig = "(hipStream_t s, unsigned grid, const FjGfArgs& g, const FjGfJob* jobs, int n_jobs, long long n_items)"
+    files, texts = [], {}
+    for c in gf_classes():
+        n = cls_name(c)
+        texts[f"gq_{n}.hip"] = (
+            "// generated by felizjueves_amd/gen_hip.py -- matrix-core gradient kernel\n"
+            '#include "../fj_device.h"\n#include "../fj_gfloop.h"\n#include "../fj_gfquad.h"\n\n'
+            f"int fj_gfquad_{n}{sig.replace('const FjGfArgs& g', 'const void* g')} {{\n"
+            f"    hipLaunchKernelGGL((fj_gfquad_k<{', '.join(map(str, c))}>), dim3(grid), dim3(GQ_THREADS), 0, s,\n"
+            "                       *static_cast<const FjGfArgs*>(g), jobs, n_jobs, n_items);\n"
+            "    return (int)hipGetLastError();\n}\n")
+        files.append(out / f"gq_{n}.hip")
+    L = ["// generated by felizjueves_amd/gen_hip.py -- matrix-core gradient launches by class", "#pragma once",
+         "// (FjGfArgs is local to each unit: its address crosses)",
+         "typedef int (*fj_gfquad_t)" + sig.replace("const FjGfArgs& g", "const void* g") + ";"]
+    L += [f"int fj_gfquad_{cls_name(c)}{sig.replace('const FjGfArgs& g', 'const void* g')};" for c in gf_classes()]
+    L += ["", "static inline fj_gfquad_t fj_gfquad_for(int la, int lb, int lc, int ld) {",
+          "    switch (((la * 4 + lb) * 4 + lc) * 4 + ld) {"]
+    L += [f"        case {((c[0] * 4 + c[1]) * 4 + c[2]) * 4 + c[3]}: return fj_gfquad_{cls_name(c)};" for c in gf_classes()]
+    L += ["        default: return nullptr;   // a class outside the stream", "    }", "}", ""]
+    texts["gq_table.h"] = "\n".join(L)
+    for fname, text in texts.items():
+        p = out / fname
+        if not p.exists() or p.read_text() != text:
+            p.write_text(text)
+    return files
+
+
 def gf_header_decls() -> str:
     return "\n".join(f"int fj_gf_{''.join(map(str, c))}(fj_stream_t stream, {GF_SIG});"
                      for c in gf_classes()) + "\n"

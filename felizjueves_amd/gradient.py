@@ -2,7 +2,7 @@
 E_2e = 1/2 tr(D (J - K/2)), RHF's Coulomb and exchange gradient terms in one
 kernel per F class (upstream `gradient/kernel_gf.py`, its stream
 `gradient/interpreted.py:293-351`, `gf_launches` / `gf_run` /
-`gf_gradient`), on the library's loop-form kernel (`fj_gf_loop` and its
+`gf_gradient`), on the library's gradient kernels (`fj_gf_loop` and its
 per-class entries `fj_gf_<la><lb><lc><ld>`).
 
     gf_launches(basis, shell_atom)            -> GfStream    the stream
@@ -30,6 +30,7 @@ from __future__ import annotations
 import ctypes as C
 import math
 from dataclasses import dataclass
+from functools import lru_cache
 
 import numpy as np
 
@@ -39,6 +40,7 @@ from .basis import Basis
 GF_LMAX = 2
 GREC = 10
 ITEMS = 2048   # work items one merged class launch aims for
+QUAD_THREADS = 256   # the width that runs the matrix-core kernel (fj_gfquad.h)
 
 
 @dataclass
@@ -120,12 +122,9 @@ def gf_launches(basis: Basis, shell_atom) -> GfStream:
 
 
 def default_threads(cls) -> int:
-    """Workgroup size of a class: 256 lanes (four wavefronts) for every
-    class. Measured per class on the three-atom s,s,p,d system and the
-    10-atom cluster at 64, 128 and 256 lanes: 256 was fastest or within 15%
-    of the fastest everywhere (the register-tiled stages have few tiles per
-    primitive quartet, so more lanes take more primitive quartets per
-    batch)."""
+    """Workgroup size of a class: 256 lanes, the width of the matrix-core
+    kernel (fj_gfquad.h); narrower ones run the loop form (the three-atom
+    s,s,p,d gradient, classes one after another: 6.1 ms against 22 ms)."""
     return 256
 
 
@@ -155,6 +154,7 @@ def _box(l1: int, l2: int) -> tuple[int, int]:
     return n, (l1 + l2 + 1) * (l1 + l2 + 2) * (l1 + l2 + 3) // 6
 
 
+@lru_cache(maxsize=None)   # `run` orders its classes by it
 def flops_per_prim_quartet(cls) -> int:
     """The arithmetic of one primitive quartet in the loop form's
     formulation: the Hermite-space weights 2 nab ncd (nu + nt) (the E
@@ -253,13 +253,18 @@ class GpuGfRunner:
             th = self.threads.get(cls, default_threads(cls))
             B = int(lib.fj_gf_batch(*[C.c_int(x) for x in cls], C.c_int(max_pq), C.c_int(th)))
             # a class of few quartets splits each quartet's primitive quartets
-            # into pieces (multiples of B) so that about ITEMS items fill the chip
+            # into pieces so that about ITEMS items fill the chip: whole rows
+            # (one bra primitive pair each) for the matrix-core kernel,
+            # multiples of the loop form's batch B otherwise
             pieces = max(1, -(-ITEMS // sum(nq)))
             q0 = 0
             for j, L in enumerate(Ls):
                 b, k = stream_.sides[L.bra], stream_.sides[L.ket]
                 n_pq = b.degree * k.degree
-                chunk = n_pq if pieces == 1 else min(n_pq, -(-(-(-n_pq // pieces)) // B) * B)
+                if th == QUAD_THREADS:
+                    chunk = -(-b.degree // pieces) * k.degree
+                else:
+                    chunk = n_pq if pieces == 1 else min(n_pq, -(-(-(-n_pq // pieces)) // B) * B)
                 jobs[j] = (rows[L.bra], rows[L.ket], b.n, k.n, b.degree, k.degree, L.diag, chunk,
                            recs[L.bra], recs[L.ket], q0)
                 q0 += nq[j] * -(-n_pq // chunk)
