@@ -63,7 +63,7 @@ def sources(lmax: int = LMAX) -> list[Path]:
     files += split
     files.append(gen_hip.write_df())   # density fitting: metric and three-center entries
     files.append(gen_hip.write_gf())   # the fused two-electron gradient's entries
-    files += gen_hip.generate_gfquad()
+    files += gen_hip.generate_gfquad() + gen_hip.generate_dfquad()
     mmd = gen_mmd.generate(MMD_LMAX, k_lmax=MMD_K_LMAX)
     gen_mmd.write_header(MMD_LMAX, MMD_K_LMAX)
     return [CSRC / "fj_runtime.hip", CSRC / "fj_mlp.hip", CSRC / "fj_plan.hip", CSRC / "fj_kloop.hip",
@@ -86,8 +86,10 @@ def _compile(src: Path, extra: list[str], force: bool = False) -> tuple[Path, fl
         deps.append(CSRC / "fj_kloop.h")
     if src.name == "fj_gfloop.hip":
         deps += [CSRC / "fj_gfloop.h", CSRC / "gen" / "gq_table.h"]
+    if src.name.startswith("dq_"):
+        deps += [CSRC / "fj_kloop.h", CSRC / "fj_dfloop.h", CSRC / "fj_dfquad.h"]
     if src.name == "fj_dfloop.hip":
-        deps.append(CSRC / "fj_dfloop.h")
+        deps += [CSRC / "fj_dfloop.h", CSRC / "gen" / "dq_table.h"]
     if src.name == "fj_kloop.hip":
         deps.append(CSRC / "fj_floop.h")
     if src.name == "fj_noalloc.hip":

@@ -24,6 +24,9 @@
 // barriers per batch, not per record pair. B is the largest that fits the LDS
 // budget, at most the cell's record pairs (fj_df_plan).
 //
+// Classes with aux shells through g run fj_dfquad.h instead, on the matrix
+// cores; this form runs h and i.
+//
 // The includer provides fj_device.h (the device one, or the CPU emulation);
 // the launchers and the per-class entries are in fj_dfloop.hip.
 #pragma once

@@ -4,6 +4,7 @@
 // call them.
 #include "fj_device.h"
 #include "fj_dfloop.h"
+#include "gen/dq_table.h"
 
 static constexpr int DF_GRID = 8192;   // workgroups per launch, at most
 
@@ -15,6 +16,9 @@ static int fj_df_launch(const FjDfArgs& g, hipStream_t s, int threads, int max_r
     if (threads % 64 || threads > 256) return FJ_ERR_THREADS;
     if (g.n_cell < 0 || g.n_aux < 0 || g.n_ao < 0) return FJ_ERR_SHAPE;
     if (g.n_cell == 0) return 0;
+    // aux shells through g on the matrix cores ((dd|g) of 9 atoms 9.7 -> 0.21
+    // ms), h and i in the loop form; `threads` shapes the loop form alone
+    if (fj_dfquad_t quad = fj_dfquad_for(g.la, g.lb, g.lc)) return quad(s, &g, g.n_cell);
     if (max_rp < 1) max_rp = DF_BMAX;
     const FjDfLds o = fj_df_plan(g.la, g.lb, g.lc, max_rp);
     const int grid = g.n_cell < DF_GRID ? g.n_cell : DF_GRID;

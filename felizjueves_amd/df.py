@@ -1,8 +1,8 @@
 """Density fitting on the GPU: the two-center Coulomb metric (P|Q) of an
 auxiliary basis (upstream `eri/density_fit/metric.py`, its kernel
 `kernel_metric.py`) and the three-center integral (mn|P) (upstream
-`eri/density_fit/eri3.py`, `kernel_eri3.py`), on the library's loop-form
-kernel (`fj_metric_loop` / `fj_eri3_loop` and their per-class entries).
+`eri/density_fit/eri3.py`, `kernel_eri3.py`), on the library's
+kernels (`fj_metric_loop` / `fj_eri3_loop` and their per-class entries).
 
     AuxBasis.from_arrays(...)              an auxiliary basis (shells through i)
     metric_classes(aux) / metric_matrix(aux)          -> (P|Q) [n_aux, n_aux]
@@ -198,7 +198,7 @@ def _p(t):
     return C.c_void_p(native.ptr(t))
 
 
-THREADS = 128   # lanes per workgroup of the DF kernel
+THREADS = 128   # lanes per workgroup of the loop-form DF kernel (aux shells h and i)
 
 
 class DfIntegrals:

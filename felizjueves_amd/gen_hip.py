@@ -805,6 +805,54 @@ def df_classes():
     return met, e3
 
 
+DQ_AUX_LMAX = 4      # aux shells of the matrix-core kernel (csrc/fj_dfquad.h)
+
+
+def dq_classes():
+    """The (la, lb, lc) of the matrix-core kernel by unit: every three-center
+    class with aux shells through g, and the metric's (lP, 0, lQ)."""
+    _, e3 = df_classes()
+    units = {}
+    for a, b, p in e3:
+        if p <= DQ_AUX_LMAX:
+            units.setdefault(f"{a}{b}", []).append((a, b, p))
+    units["metric"] = [(p, 0, q) for p in range(1, DQ_AUX_LMAX + 1) for q in range(p, DQ_AUX_LMAX + 1)]
+    return units
+
+
+def generate_dfquad(out: Path = GEN) -> list[Path]:
+    """dq_<unit>.hip, launches of the matrix-core density-fitting kernel, and
+    dq_table.h, their dispatch."""
+    out.mkdir(parents=True, exist_ok=True)
+    files, texts = [], {}
+    sig = "(hipStream_t s, const void* g, int n_cell)"   # FjDfArgs is local to each unit
+    for name, classes in dq_classes().items():
+        L = ["// generated by felizjueves_amd/gen_hip.py -- matrix-core density-fitting kernel",
+             '#include "../fj_device.h"', '#include "../fj_dfloop.h"', '#include "../fj_dfquad.h"', ""]
+        for a, b, p in classes:
+            L += [f"int fj_dfquad_{a}{b}{p}{sig} {{",
+                  f"    constexpr int per = Dq<{a}, {b}, {p}>::CW;",
+                  f"    hipLaunchKernelGGL((fj_dfquad_k<{a}, {b}, {p}>), dim3((unsigned)((n_cell + per - 1) / per)),",
+                  "                       dim3(DQ_THREADS), 0, s, *static_cast<const FjDfArgs*>(g));",
+                  "    return (int)hipGetLastError();", "}", ""]
+        texts[f"dq_{name}.hip"] = "\n".join(L)
+        files.append(out / f"dq_{name}.hip")
+    every = [c for classes in dq_classes().values() for c in classes]
+    L = ["// generated by felizjueves_amd/gen_hip.py -- matrix-core density-fitting launches by class", "#pragma once",
+         f"typedef int (*fj_dfquad_t){sig};"]
+    L += [f"int fj_dfquad_{a}{b}{p}{sig};" for a, b, p in every]
+    L += ["", "static inline fj_dfquad_t fj_dfquad_for(int la, int lb, int lc) {",
+          "    switch ((la * 8 + lb) * 8 + lc) {"]
+    L += [f"        case {(a * 8 + b) * 8 + p}: return fj_dfquad_{a}{b}{p};" for a, b, p in every]
+    L += ["        default: return nullptr;   // on the loop form", "    }", "}", ""]
+    texts["dq_table.h"] = "\n".join(L)
+    for fname, text in texts.items():
+        p = out / fname
+        if not p.exists() or p.read_text() != text:
+            p.write_text(text)
+    return files
+
+
 METRIC_SIG = ("int threads, int n_pair, int n_rec, int n_aux, const double* A, const double* alpha,"
               " const double* s_aux, const int* p_rec0, const int* p_rec1, const int* q_rec0,"
               " const int* q_rec1, const int* off_p, const int* off_q, double* metric")
