@@ -321,6 +321,8 @@ class FockBuilder:
     independent systems in the same launches: every class pair of every
     system is one launch per tier, each work item naming its system."""
 
+    weights = (2.0, -0.5)   # of the Coulomb and exchange blocks: J - K/2 (hjk.HJKBuild takes J or K)
+
     def __init__(self, basis: Basis, D: np.ndarray, *, tau: float = 1e-12, threads=64,
                  mixed: bool = False, fp32_error: float = 1e-11, selector=None,
                  lane_flops=None, fp32_bound: float | None = None, planner: str = "auto",
@@ -872,7 +874,7 @@ class FockBuilder:
             c = L.coop
             native.call_fc(L.cls, c.parts, L.bra.side, L.ket.side, c.dev[0], c.work.shape[0], c.dev[1],
                            c.dev[2], L.tier_dev if L.precision == MIXED else None, sys, L.diag,
-                           self.tau, stream)
+                           self.tau, stream, self.weights)
             return
         if L.precision == MIXED:
             native.call_fxm(L.cls, L.threads, L.bra.side, L.ket.side, L.work_dev, L.work.shape[0],

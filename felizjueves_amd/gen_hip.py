@@ -1730,6 +1730,7 @@ def emit_coop(cls) -> str:
                 if (!({here})) continue;
                 int s0, s1, i, j;
                 B::of(t % {NO}, s0, s1, i, j);
+                if (((s0 == 0 && s1 == 1) || s0 == 2 ? cj : ck) == 0.0) continue;   // a J or K build
                 const double x = B::template sum<{XS}>(X + u * {NAB * XS}, wd + u * {NO}, s0, s1, i, j, 0, {na});
                 {store}
             }}
@@ -1758,6 +1759,7 @@ def emit_coop(cls) -> str:
                 const double x = acc[u];
                 int s0, s1, i, j;
                 B::of(lane + 64 * u, s0, s1, i, j);
+                if (((s0 == 0 && s1 == 1) || s0 == 2 ? cj : ck) == 0.0) continue;
                 {store}
             }}
 """
@@ -1767,7 +1769,7 @@ template <bool MIXED>
 __device__ __forceinline__ void fj_citem_{name}(const FjFArgs& a, int it, bool f32, int part, int parts,
                                              double* __restrict__ bsh, double* __restrict__ bnd_,
                                              double* __restrict__ wt, double* __restrict__ fab,
-                                             FjCoopKets<{NQ}>* __restrict__ K_) {{
+                                             FjCoopKets<{NQ}>* __restrict__ K_, double cj, double ck) {{
     typedef FjCoopBlocks<{na}, {nb}, {nc}, {nd}> B;
     static_assert(B::N == {NO}, "elements of the F blocks");
     const int4 w = a.work[it];
@@ -1842,7 +1844,7 @@ __device__ __forceinline__ void fj_citem_{name}(const FjFArgs& a, int it, bool f
                 if (a.diag && k == bra) deg *= 0.5;
                 const int ro = s0 == 0 ? oa : s0 == 1 ? ob : oc, co = s1 == 1 ? ob : s1 == 2 ? oc : od;
                 const bool coul = (s0 == 0 && s1 == 1) || s0 == 2;
-                wd[t] = (coul ? 2.0 * deg : -0.5 * deg) * S.D[(size_t)(ro + i) * n_ao + co + j];
+                wd[t] = (coul ? cj : ck) * deg * S.D[(size_t)(ro + i) * n_ao + co + j];
             }}
 {phase_cd}            fj_wave_sync();
         }}
@@ -1855,12 +1857,12 @@ __device__ __forceinline__ void fj_citem_{name}(const FjFArgs& a, int it, bool f
 }}
 
 template <bool MIXED>
-__global__ void __launch_bounds__(FJ_COOP_THREADS, {h["wgs"]}) fj_c_{name}_k(FjFArgs a, const int* parent) {{
+__global__ void __launch_bounds__(FJ_COOP_THREADS, {h["wgs"]}) fj_c_{name}_k(FjFArgs a, const int* parent, double cj, double ck) {{
     __shared__ double bsh[FJ_MAX_PRIM_PAIRS * FJ_SREC], bnd[{4 * NQ * REG}], wt[{4 * WT}], fab[{NAB}];
     __shared__ FjCoopKets<{NQ}> K[FJ_COOP_WAVES];
     const int it = (int)blockIdx.x;
     fj_citem_{name}<MIXED>(a, it, MIXED && !fj_item_fp64(a, parent[it]), (int)blockIdx.y, (int)gridDim.y, bsh, bnd, wt,
-                        fab, K);
+                        fab, K, cj, ck);
 }}
 """)
     return E.text()
@@ -1869,10 +1871,10 @@ __global__ void __launch_bounds__(FJ_COOP_THREADS, {h["wgs"]}) fj_c_{name}_k(FjF
 def coop_entry(cls) -> str:
     """fj_fc_<cls>, the cooperative launch of a builder work list."""
     n = cls_name(cls)
-    return (f"int fj_claunch_{n}_mx(hipStream_t s, dim3 grid, const FjFArgs& a, const int* parent);\n\n"
+    return (f"int fj_claunch_{n}_mx(hipStream_t s, dim3 grid, const FjFArgs& a, const int* parent, double cj, double ck);\n\n"
             f'extern "C" int fj_fc_{n}(hipStream_t s, int parts, const FjSide* bra, const FjSide* ket,\n'
             "                        const int* work, int n_work, const int* ket_list, const int* parent,\n"
-            "                        const int* tier, const FjSys* sys, int diag, double tau) {\n"
+            "                        const int* tier, const FjSys* sys, int diag, double tau, double cj, double ck) {\n"
             "    if (!bra || !ket || !work || !sys || !ket_list || (tier && !parent)) return FJ_ERR_ARG;\n"
             "    if (parts < 1 || parts > 64) return FJ_ERR_ARG;\n"
             "    if (n_work <= 0 || ket->n <= 0) return 0;\n"
@@ -1885,8 +1887,8 @@ def coop_entry(cls) -> str:
             "    a.ws = nullptr; a.ws_doubles = 0; a.n_bx = n_work; a.n_items = n_work;\n"
             "    a.n_fp64 = 0; a.tier = tier;\n"
             "    const dim3 grid((unsigned)n_work, (unsigned)parts);\n"
-            f"    if (tier) return fj_claunch_{n}_mx(s, grid, a, parent);\n"
-            f"    hipLaunchKernelGGL(fj_c_{n}_k<false>, grid, dim3(FJ_COOP_THREADS), 0, s, a, parent);\n"
+            f"    if (tier) return fj_claunch_{n}_mx(s, grid, a, parent, cj, ck);\n"
+            f"    hipLaunchKernelGGL(fj_c_{n}_k<false>, grid, dim3(FJ_COOP_THREADS), 0, s, a, parent, cj, ck);\n"
             "    return (int)hipGetLastError();\n}\n")
 
 
@@ -1901,8 +1903,8 @@ def generate_coop(classes, out: Path = GEN) -> list[Path]:
         texts = {f"c_{n}.h": emit_coop(cls),
                  f"c_{n}.hip": gen + f'#include "c_{n}.h"\n\n' + coop_entry(cls),
                  f"c_{n}_mx.hip": gen + f'#include "c_{n}.h"\n\n'
-                 f"int fj_claunch_{n}_mx(hipStream_t s, dim3 grid, const FjFArgs& a, const int* parent) {{\n"
-                 f"    hipLaunchKernelGGL(fj_c_{n}_k<true>, grid, dim3(FJ_COOP_THREADS), 0, s, a, parent);\n"
+                 f"int fj_claunch_{n}_mx(hipStream_t s, dim3 grid, const FjFArgs& a, const int* parent, double cj, double ck) {{\n"
+                 f"    hipLaunchKernelGGL(fj_c_{n}_k<true>, grid, dim3(FJ_COOP_THREADS), 0, s, a, parent, cj, ck);\n"
                  f"    return (int)hipGetLastError();\n}}\n"}
         for fname, text in texts.items():
             p = out / fname
@@ -1935,7 +1937,7 @@ def write_coop_header(classes) -> None:
     decl = "\n".join(
         f"int fj_fc_{cls_name(c)}(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,\n"
         f"    const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,\n"
-        f"    const FjSys* sys, int diag, double tau);" for c in classes) + "\n"
+        f"    const FjSys* sys, int diag, double tau, double cj, double ck);" for c in classes) + "\n"
     cur = HEADER.read_text()
     i, j = cur.index(COOP_BEGIN), cur.index(COOP_END)
     text = cur[:i + len(COOP_BEGIN)] + "\n" + decl + cur[j:]

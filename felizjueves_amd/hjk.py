@@ -345,17 +345,24 @@ STREAMS = 4   # streams of a staged build (hardware queues per process on the MI
 
 
 class HJKBuild:
-    """A split J or K build staged on the device for repeated use: the
-    plan's launch arguments on the device (each (batch, orientation) side
-    once, D and its block maxima once), `run()` issuing every launch into
-    one n_ao x n_ao accumulator on one stream, and `capture()` / `replay()`
-    the same build as one HIP graph (the accumulator cleared by torch's fill
-    kernel, no memset node). The build is for the density it was staged
-    with; the result is walk_hjk's (nothing closed or mirrored).
+    """A split J or K build staged on the device for repeated use: the tables
+    on the device once, `run()` issuing every launch into one n_ao x n_ao
+    accumulator, and `capture()` / `replay()` the same build as one HIP graph
+    (the accumulator cleared by torch's fill kernel, no memset node). The
+    build is for the density it was staged with; the result is walk_hjk's.
 
-    `quartets_computed` and `flops` count the quartets that pass the
-    in-kernel screen (G_ab G_cd times the density block, D_cd for J and D_bd
-    for K) and their algorithmic FLOPs (hgp.cost of the kernel's class)."""
+    Without a `plan` the build takes the fused builder's unique quartets
+    through its quartet-cooperative kernels with the Coulomb or the exchange
+    blocks alone (45 launches), at a screen that keeps every quartet the
+    split stream's keeps: three atoms s,s,p,d, four streams, one graph, J
+    43.1 -> 0.50 ms. A given `plan` runs launch by launch through the split
+    kernels, as planned (4,761 launches there: each (batch, orientation) side,
+    D and its block maxima on the device once).
+
+    `quartets_computed` and `flops` count the split stream's quartets that
+    pass its in-kernel screen (G_ab G_cd times the density block, D_cd for J
+    and D_bd for K) and their algorithmic FLOPs (hgp.cost of the kernel's
+    class)."""
 
     def __init__(self, basis: Basis, D, *, tau: float = 1e-12, screen: str = "j",
                  threads: int = 64, plan: HPlan | None = None):
@@ -367,8 +374,40 @@ class HJKBuild:
             raise ValueError("the plan is for the other screen")
         self.basis, self.screen, self.threads = basis, screen, threads
         self.kind = "hj" if screen == "j" else "hk"
+        self.graph = None
+        n_q, fl = 0, 0.0
+        for L in self.plan.launches:
+            bra, ket = self.plan.batches[L.bra], self.plan.batches[L.ket]
+            gb = np.array([p.G for p in bra.pairs])
+            gk = np.array([q.G for q in ket.pairs])
+            if screen == "j":
+                dm = np.array([self.plan.dmax[q.a, q.b] for q in ket.pairs])[None, :]
+            else:
+                dm = self.plan.dmax[np.array([p.b for p in bra.pairs])[:, None],
+                                    np.array([q.b for q in ket.pairs])[None, :]]
+            live = int(np.count_nonzero(gb[:, None] * gk[None, :] * dm >= self.plan.tau))
+            n_q += live
+            fl += live * cost(L.cls).flops(bra.degree, ket.degree)
+        self.quartets_computed, self.flops = n_q, fl
+        self.builder = None
+        if plan is None:
+            from .fock import FockBuilder
+            # the fused screen tests G_ab G_cd max(2 D_ab, 2 D_cd, D_ac / 2, ..): at
+            # tau / 2 max|D| it and the density-free one pass what the split one does
+            t = float(tau) / (2.0 * max(1.0, float(np.abs(D).max())))
+            self.builder = FockBuilder(basis, D, tau=t, coop=True)
+            self.builder.weights = (2.0, 0.0) if screen == "j" else (0.0, 1.0)
+            self.builder.to_device()
+            self._D = native.to_dev(np.ascontiguousarray(D))
+            self.X = self.builder.F
+            return
+        self._stage(D)
+
+    def _stage(self, D) -> None:
+        """Every launch's arguments on the device (a given plan)."""
+        from . import native
         self.runner = GpuHJKRunner()
-        plan = self.plan
+        basis, plan = self.basis, self.plan
         dD = native.to_dev(np.ascontiguousarray(D.ravel()))
         dDsh = native.to_dev(np.ascontiguousarray(plan.dmax.ravel()))
         sides: dict = {}
@@ -378,7 +417,7 @@ class HJKBuild:
                 sides[(bi, sw)] = {k: (native.to_dev(v) if isinstance(v, np.ndarray) else v)
                                    for k, v in side_records(basis, plan, plan.batches[bi], sw).items()}
             return sides[(bi, sw)]
-        self.staged, n_q, fl = [], 0, 0.0
+        self.staged = []
         for L in plan.launches:
             (bi, bs), (ki, ks) = kernel_sides(L)
             b, k = side(bi, bs), side(ki, ks)
@@ -392,20 +431,7 @@ class HJKBuild:
             if k["lb"]:
                 a["CD"] = k["sep"]
             self.staged.append(((self.kind, L.cls), a))
-            bra, ket = plan.batches[L.bra], plan.batches[L.ket]
-            gb = np.array([p.G for p in bra.pairs])
-            gk = np.array([q.G for q in ket.pairs])
-            if screen == "j":
-                dm = np.array([plan.dmax[q.a, q.b] for q in ket.pairs])[None, :]
-            else:
-                dm = plan.dmax[np.array([p.b for p in bra.pairs])[:, None],
-                               np.array([q.b for q in ket.pairs])[None, :]]
-            live = int(np.count_nonzero(gb[:, None] * gk[None, :] * dm >= plan.tau))
-            n_q += live
-            fl += live * cost(L.cls).flops(bra.degree, ket.degree)
-        self.quartets_computed, self.flops = n_q, fl
         self.X = self.runner.zeros(basis.n_ao)
-        self.graph = None
 
     def run(self, n_streams: int = 1):
         """Every launch of the build into X (cleared first); returns X (on
@@ -415,6 +441,8 @@ class HJKBuild:
         library keeps one workspace per stream for the classes that need
         one, so launches on different streams may overlap)."""
         import torch
+        if self.builder is not None:
+            return self.builder.build(self._D, n_streams=n_streams)
         self.X.zero_()
         if n_streams <= 1:
             for kern, a in self.staged:
@@ -437,6 +465,9 @@ class HJKBuild:
         eager build on the same streams: the library's workspace is per
         stream and allocated on first use, which a capture may not do."""
         import torch
+        if self.builder is not None:
+            self.graph = self.builder.capture(self._D, n_streams=n_streams)
+            return self.graph
         g = torch.cuda.CUDAGraph()
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())

@@ -166,15 +166,17 @@ def coop_batch(cls) -> int:
 
 
 def call_fc(cls, parts: int, bra: FjSide, ket: FjSide, work, n_work: int, ket_list, parent, tier, sys,
-            diag: int, tau: float, stream=None) -> None:
+            diag: int, tau: float, stream=None, weights=(2.0, -0.5)) -> None:
     """One quartet-cooperative launch fj_fc_<cls>: `work`, `ket_list` as for
     call_fx, each item over `parts` workgroups; with `tier` (a device int32
-    array) item i in tier[parent[i]], else in FP64."""
+    array) item i in tier[parent[i]], else in FP64; `weights` of the Coulomb
+    and the exchange blocks (J - K/2)."""
     fn = getattr(lib(), "fj_fc_" + "".join(map(str, cls)))
     fn.restype = C.c_int
     rc = fn(C.c_void_p(stream_handle(stream)), C.c_int(parts), C.byref(bra), C.byref(ket),
             C.c_void_p(ptr(work)), C.c_int(n_work), C.c_void_p(ptr(ket_list)), C.c_void_p(ptr(parent)),
-            C.c_void_p(ptr(tier)), C.c_void_p(ptr(sys)), C.c_int(diag), C.c_double(tau))
+            C.c_void_p(ptr(tier)), C.c_void_p(ptr(sys)), C.c_int(diag), C.c_double(tau),
+            *[C.c_double(w) for w in weights])
     check(rc, fn.__name__)
 
 

@@ -1256,144 +1256,146 @@ int fj_fxm_3333(fj_stream_t stream, int threads, const FjSide* bra, const FjSide
  * workgroups. ket_list is required; any number of entries per item is taken
  * fj_fc_batch(class) at a time (fj_fc_batch: 0 for a class without this
  * form). With `tier` (per planned item, 0 FP64 / 1 FP32) item i runs in
- * tier[parent[i]], else in FP64. No workspace. */
+ * tier[parent[i]], else in FP64. cj and ck weight the Coulomb and the exchange
+ * blocks: F closed (F + F^T) is G for (2, -1/2), J for (2, 0), K for (0, 1).
+ * No workspace. */
 int fj_fc_batch(int la, int lb, int lc, int ld);
 /* BEGIN COOPERATIVE CLASSES (written by felizjueves_amd/gen_hip.py) */
 int fj_fc_0000(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0001(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0002(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0010(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0011(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0012(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0020(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0021(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0022(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0101(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0102(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0110(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0111(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0112(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0120(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0121(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0122(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0202(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0210(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0211(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0212(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0220(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0221(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_0222(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1010(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1011(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1012(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1020(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1021(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1022(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1111(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1112(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1120(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1121(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1122(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1212(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1220(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1221(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_1222(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_2020(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_2021(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_2022(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_2121(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_2122(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 int fj_fc_2222(fj_stream_t stream, int parts, const FjSide* bra, const FjSide* ket,
     const int* work, int n_work, const int* ket_list, const int* parent, const int* tier,
-    const FjSys* sys, int diag, double tau);
+    const FjSys* sys, int diag, double tau, double cj, double ck);
 /* END COOPERATIVE CLASSES */
 
 /* The MMD families, one entry per class, each with the upstream kernel's

@@ -58,7 +58,7 @@ int main(int argc, char** argv) {
                 for (unsigned x = 0; x < gridDim.x; ++x) {
                     if (t == 0) blockIdx = {x, y, 0};
                     bar.arrive_and_wait();
-                    KERNEL<true>(a, parent);
+                    KERNEL<true>(a, parent, 2.0, -0.5);
                     bar.arrive_and_wait();
                 }
         });

@@ -93,3 +93,29 @@ def test_cooperative_entry_refuses():
         with pytest.raises(native.FjError):
             native.call_fc(L.cls, parts, L.bra.side, L.ket.side, d[0], 1, kets, d[2], None, sys, L.diag, fb.tau)
     assert native.coop_batch((0, 0, 3, 3)) == 0 and native.coop_batch((0, 0, 0, 0)) > 0
+
+
+@pytest.mark.parametrize("screen", ["j", "k"])
+@pytest.mark.parametrize("tau,n_streams", [(0.0, 1), (1e-12, 4)])
+def test_split_build_without_a_plan(screen, tau, n_streams):
+    """hjk.HJKBuild on the Coulomb or exchange blocks alone, eager and three
+    graph replays with eager builds between them, against the oracle's sweep
+    of every ordered quartet (at tau, at most 2e4 quartets below tau / 2 each
+    are dropped, of either sign: 7e-11 together)."""
+    _need_gpu()
+    from felizjueves_amd import hjk
+    from felizjueves_amd.systems import config1
+    from oracle import oracle as O
+    s = config1()
+    ref = O.fock_ordered(s.basis, s.D)[screen == "k"]
+    b = hjk.HJKBuild(s.basis, s.D, tau=tau, screen=screen)
+    got = [b.run(n_streams).cpu().numpy()]
+    b.capture(n_streams)
+    for _ in range(3):
+        got.append(b.replay().cpu().numpy())
+        got.append(b.run(n_streams).cpu().numpy())
+    for X in got:
+        assert np.abs(X - ref).max() <= 1e-12 * max(1.0, np.abs(ref).max()) + 100 * tau
+        assert np.abs(X - X.T).max() == 0.0   # closed
+    print(screen, tau, "max|X - sweep|", max(np.abs(X - ref).max() for X in got), flush=True)
+    assert b.quartets_computed > 0 and b.flops > 0
