@@ -48,6 +48,7 @@ def sources(lmax: int = LMAX) -> list[Path]:
         if not p.exists() or p.read_text() != text:
             p.write_text(text)
         files.append(p)
+        files += gen_hip.generate_fquad(loop)   # and the matrix-core kernel of their work-list launches
     built = set(classes) | set(loop)
     gen_hip.write_header(tuple(c for c in builder_classes(LOOP_LMAX) if c in built))
     gen_hip.write_coop_header(classes)
@@ -90,8 +91,11 @@ def _compile(src: Path, extra: list[str], force: bool = False) -> tuple[Path, fl
         deps += [CSRC / "fj_kloop.h", CSRC / "fj_dfloop.h", CSRC / "fj_dfquad.h"]
     if src.name == "fj_dfloop.hip":
         deps += [CSRC / "fj_dfloop.h", CSRC / "gen" / "dq_table.h"]
+    if src.name.startswith("fq_"):
+        deps += [CSRC / "fj_fitem.h", CSRC / "fj_fquad.h"]
+        extra = [*extra, "-fconstexpr-steps=50000000"]   # the index tables of the (ff| classes
     if src.name == "fj_kloop.hip":
-        deps.append(CSRC / "fj_floop.h")
+        deps += [CSRC / "fj_fitem.h", CSRC / "fj_floop.h", CSRC / "gen" / "fq_table.h"]
     if src.name == "fj_noalloc.hip":
         deps.append(CSRC / "gen" / "f_any_table.h")
     if not force and obj.exists() and all(obj.stat().st_mtime >= d.stat().st_mtime

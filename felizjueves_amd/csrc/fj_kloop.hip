@@ -1,11 +1,13 @@
 // fj_kloop.hip -- launchers of the loop-form MMD kernels (fj_kloop.h): K
 // (the entries fj_k_<la><lc><lb><ld> of the classes with an f shell and the
 // generic fj_k_loop) and Schwarz (fj_schwarz_<la><lb> past la + lb = 4 and
-// the generic fj_schwarz_loop) and the fused F kernel of the classes with
-// an f shell (their fj_f_ / fj_fx_ / fj_fxm_ entries, generated).
+// the generic fj_schwarz_loop) and the fused F kernels of the classes with
+// an f shell (their fj_f_ entries in loop form; fj_fx_ / fj_fxm_, with a work
+// list, on fj_fquad.h; generated).
 #include "fj_device.h"
 #include "fj_kloop.h"
 #include "fj_floop.h"
+#include "gen/fq_table.h"
 
 // x[0 .. n) = 0, grid-stride (vector stores).
 __global__ void fj_kl_zero_k(double* __restrict__ x, long long n) {
@@ -90,12 +92,19 @@ int fj_floop_launch(hipStream_t s, int la, int lb, int lc, int ld, int threads, 
     if (threads <= 0) threads = FJ_DEFAULT_THREADS;
     if (threads % 64 || threads > FJ_MAX_THREADS) return FJ_ERR_THREADS;
     if (n_blocks <= 0 || a.ket.n <= 0) return 0;
-    // with a work list, each item's kets are cut into up to `threads` slices,
-    // one workgroup each, so that a launch of few long items still fills the
-    // chip (a workgroup takes its kets one after another)
-    const int split = a.work ? std::max(1, std::min(threads, FJ_FL_WORKGROUPS / n_blocks)) : 0;
-    const dim3 grid((unsigned)n_blocks,
-                    a.work ? (unsigned)split : (unsigned)((a.ket.n + threads - 1) / threads));
+    // A work list (the Fock builder) runs on the matrix-core kernel, each item's
+    // kets cut into up to `threads` slices, one workgroup each, so that a launch
+    // of few long items still fills the chip (a workgroup takes its kets one
+    // after another): 4 atoms with f shells 38.0 -> 9.7 ms against the loop
+    // form. Launches without one, of the reference's argument lists, whose
+    // slices are fixed at `threads` kets, stay on the loop form.
+    if (a.work) {
+        const fj_fquad_t quad = fj_fquad_for(la, lb, lc, ld);
+        if (!quad) return FJ_ERR_ARG;
+        const int split = std::max(1, std::min(threads, FJ_FL_WORKGROUPS / n_blocks));
+        return quad(s, dim3((unsigned)n_blocks, (unsigned)split), threads, a);
+    }
+    const dim3 grid((unsigned)n_blocks, (unsigned)((a.ket.n + threads - 1) / threads));
     a.n_bx = (int)grid.x;
     a.n_items = (int)(grid.x * grid.y);
     // the batched kernel where B >= 2 primitive quartets fit its LDS budget,

@@ -970,6 +970,46 @@ def generate_gfquad(out: Path = GEN) -> list[Path]:
     return files
 
 
+def fq_units(classes):
+    """The classes of the matrix-core F kernel (csrc/fj_fquad.h) by unit: one
+    bra pair class each, (3, 3) kets apart."""
+    units = {}
+    for c in classes:
+        units.setdefault("{}{}".format(*c[:2]) + ("_ff" if c[2:] == (3, 3) else ""), []).append(c)
+    return units
+
+
+def generate_fquad(classes, out: Path = GEN) -> list[Path]:
+    """fq_<unit>.hip, launches of the matrix-core F kernel of the classes with
+    an f shell, and fq_table.h, their dispatch."""
+    out.mkdir(parents=True, exist_ok=True)
+    sig = "(hipStream_t s, dim3 grid, int span, const FjFArgs& a)"
+    files, texts = [], {}
+    for name, cs in fq_units(classes).items():
+        L = ["// generated by felizjueves_amd/gen_hip.py -- matrix-core F kernel",
+             '#include "../fj_device.h"', '#include "../fj_fquad.h"', ""]
+        for c in cs:
+            L += [f"int fj_fquad_{cls_name(c)}{sig} {{",
+                  f"    grid.z = Fq<{', '.join(map(str, c))}>::Z;",
+                  f"    hipLaunchKernelGGL((fj_fquad_k<{', '.join(map(str, c))}>), grid, dim3(FQ_THREADS), 0, s, span, a);",
+                  "    return (int)hipGetLastError();", "}", ""]
+        texts[f"fq_{name}.hip"] = "\n".join(L)
+        files.append(out / f"fq_{name}.hip")
+    L = ["// generated by felizjueves_amd/gen_hip.py -- matrix-core F launches by class", "#pragma once",
+         f"typedef int (*fj_fquad_t){sig};"]
+    L += [f"int fj_fquad_{cls_name(c)}{sig};" for c in classes]
+    L += ["", "static inline fj_fquad_t fj_fquad_for(int la, int lb, int lc, int ld) {",
+          "    switch (((la * 4 + lb) * 4 + lc) * 4 + ld) {"]
+    L += [f"        case {((c[0] * 4 + c[1]) * 4 + c[2]) * 4 + c[3]}: return fj_fquad_{cls_name(c)};" for c in classes]
+    L += ["        default: return nullptr;   // a class without an f shell", "    }", "}", ""]
+    texts["fq_table.h"] = "\n".join(L)
+    for fname, text in texts.items():
+        p = out / fname
+        if not p.exists() or p.read_text() != text:
+            p.write_text(text)
+    return files
+
+
 def gf_header_decls() -> str:
     return "\n".join(f"int fj_gf_{''.join(map(str, c))}(fj_stream_t stream, {GF_SIG});"
                      for c in gf_classes()) + "\n"
