@@ -119,3 +119,5 @@ def test_split_build_without_a_plan(screen, tau, n_streams):
         assert np.abs(X - X.T).max() == 0.0   # closed
     print(screen, tau, "max|X - sweep|", max(np.abs(X - ref).max() for X in got), flush=True)
     assert b.quartets_computed > 0 and b.flops > 0
+    with pytest.raises(RuntimeError):   # a width the split kernels refuse is refused still
+        hjk.HJKBuild(s.basis, s.D, tau=tau, screen=screen, threads=100).run()
