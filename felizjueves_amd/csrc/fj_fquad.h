@@ -28,8 +28,8 @@
 // summed index is multiplied by zero (bit 30 of a table entry).
 //
 // Bound, for the d and f pairs, by the matrix cores and the FP64 instructions
-// that form their operands ((ff|ff): 7.4 of them a step, the cores busy for a
-// third of the time), for the low classes by the latency of a workgroup (Boys
+// that form their operands ((ff|ff): 7.4 VALU instructions a step, the cores busy
+// 27% of the time), for the low classes by the latency of a workgroup (Boys
 // function, tower levels, digestion) and by new code for every launch. Measured
 // on MI355X, 4 atoms s,s,p,d,f, 4 streams, 18,274 quartets (1.3 million
 // primitive quartets with an f): the build 38.0 -> 9.7 ms; another of 4 atoms
