@@ -335,7 +335,7 @@ def _aux_even_tempered(coords, ls=(0, 1, 2, 3, 4), n=4, a0=0.3, ratio=2.5):
 
 def df_block(cpu: bool = True) -> dict:
     """The density-fitting integrals (df.py: the metric (P|Q) and the
-    three-center (mn|P) on the loop-form kernel) on the upstream fixtures
+    three-center (mn|P) on the matrix-core kernel) on the upstream fixtures
     (H2O cc-pVTZ-JKFIT metric, 166 aux functions; H2O STO-3G x JKFIT
     three-center) with max|d| against libcint, and on the 10-atom cluster
     with a synthetic even-tempered s..g aux set (20 shells per atom,
@@ -599,7 +599,7 @@ def c4_block(a) -> None:
 def cof_block(a) -> None:
     """The f workload: CO/cc-pVTZ (f shells on both atoms), the Fock build
     through (ff|ff) -- HGP kernels through (dd|dd), the classes with an f
-    shell on the loop-form kernel -- and the MMD families through f (J
+    shell on the matrix-core kernel -- and the MMD families through f (J
     chain, K, Schwarz), each timed on the device and checked against
     libcint's vj / vk of the committed fixture."""
     import torch
@@ -621,7 +621,7 @@ def cof_block(a) -> None:
     J, K = cj.run(Dd).cpu().numpy(), ck.run(Dd).cpu().numpy()
     torch.cuda.synchronize()
     out = {
-        "metric": "Fock builds/s, CO/cc-pVTZ (f shells; f classes on the loop-form kernel)",
+        "metric": "Fock builds/s, CO/cc-pVTZ (f shells; f classes on the matrix-core kernel)",
         "value": a.steps / t, "unit": "Fock builds/s", "n_gpus": 1, "steps": a.steps,
         "warmup": a.warmup, "ms_per_step": 1e3 * t / a.steps, "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f64", "data": "committed fixture",
@@ -736,7 +736,7 @@ def main() -> None:
                     default="c2",
                     help="c4d: the 64-molecule batch (8-80 atoms, seeds 4+i) with s,s,p,d shells "
                          "(with its f shells, 45,402 AOs, one build would take minutes on the "
-                         "loop-form f kernels); cof: CO/cc-pVTZ through f (the loop-form kernels); c4f: "
+                         "matrix-core f kernels); cof: CO/cc-pVTZ through f (the matrix-core kernels); c4f: "
                          "single C4 molecules with and without their f shells; c4f-batch: "
                          "chosen C4 molecules with f in one batch builder; gradient: the fused "
                          "two-electron gradient block alone; split-df: the split J / K and "
