@@ -402,3 +402,24 @@ extern "C" int fj_tier_select_jobs(hipStream_t s, int n_jobs, const FjTierJob* j
                        n_feat, W);
     return (int)hipGetLastError();
 }
+
+// A cooperative item's tier: FP32 where every planned item under it is. A
+// thread per item; the planned items under one are few (one to the chunks a
+// quartet was split into).
+__global__ void __launch_bounds__(256) fj_tier_cover_k(int n, const int* __restrict__ off,
+                                                       const int* __restrict__ items,
+                                                       const int* __restrict__ tier, int* __restrict__ out) {
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n) return;
+    int all = 1;
+    for (int e = off[i]; e < off[i + 1]; ++e) all &= tier[items[e]];
+    out[i] = all;
+}
+
+extern "C" int fj_tier_cover(hipStream_t s, int n, const int* off, const int* items, const int* tier, int* out) {
+    if (n < 0) return FJ_ERR_SHAPE;
+    if (n == 0) return 0;
+    if (!off || !items || !tier || !out) return FJ_ERR_ARG;
+    hipLaunchKernelGGL(fj_tier_cover_k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, off, items, tier, out);
+    return (int)hipGetLastError();
+}

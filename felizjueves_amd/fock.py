@@ -137,7 +137,9 @@ class CoopItems:
     ket_list: np.ndarray
     parent: np.ndarray
     parts: int
-    dev: tuple = ()           # (work, ket_list, parent) on the device
+    dev: tuple = ()           # (work, ket_list, identity) on the device
+    cover: tuple = ()         # MIXED: (offsets, planned items) of coop_cover
+    tier: object = None       # MIXED: per-item tiers on the device, from the planned items'
 
 
 def coop_items(work: np.ndarray, ket_list: np.ndarray, batch: int):
@@ -159,6 +161,42 @@ def coop_items(work: np.ndarray, ket_list: np.ndarray, batch: int):
     hi = k0[rep] + (j + 1) * n[rep] // pieces[rep]
     out = np.stack([w[parent[rep], 0], lo, w[parent[rep], 2] & 0xffff, hi], axis=1)
     return out.astype(np.int32), (ket_list[first] & 0x1ffff).astype(np.int32), parent[rep].astype(np.int32)
+
+
+def coop_cover(work: np.ndarray, ket_list: np.ndarray, items):
+    """(offsets [n + 1], planned items) of the cooperative `items` (work, ket
+    list, parent): every planned item that holds some chunk of an item's
+    quartets. The error rule clears a planned item's chunks for FP32, so an
+    item may run in FP32 only where all of these may."""
+    cw, ck, parent = items
+    n = len(cw)
+    w = work.astype(np.int64)
+    if not (ket_list >> 17).any() and not (w[:, 2] >> 16).any():   # no quartet is split
+        return np.arange(n + 1, dtype=np.int32), parent.astype(np.int32)
+
+    def entries(lo, hi):   # (range, entry) of the entries of the ranges [lo, hi)
+        r = np.repeat(np.arange(len(lo)), hi - lo)
+        return r, np.arange(len(r)) + np.repeat(lo - (np.cumsum(hi - lo) - (hi - lo)), hi - lo)
+    # each list entry's cooperative item: first chunks by their place, later
+    # ones by their quartet (bra, ket), among the first chunks of split kets
+    first = np.nonzero((ket_list & (0x7f << 17)) == 0)[0]
+    later = np.nonzero(ket_list & (0x7f << 17))[0]
+    r, at = entries(cw[:, 1].astype(np.int64), cw[:, 3].astype(np.int64))
+    of = np.empty(len(ket_list), dtype=np.int64)
+    of[first[at]] = r
+    whole_bra = np.nonzero(((w[:, 2] >> 16) & 0xff) == 0)[0]
+    r, at = entries(w[whole_bra, 1], w[whole_bra, 3])
+    quartet = np.empty(len(ket_list), dtype=np.int64)
+    quartet[at] = w[whole_bra[r], 0] << 17
+    quartet |= ket_list & 0x1ffff
+    split = first[ket_list[first] >> 24 != 0]
+    split = split[np.argsort(quartet[split])]
+    of[later] = of[split[np.searchsorted(quartet[split], quartet[later])]]
+    r, at = entries(w[:, 1], w[:, 3])
+    pair = of[at] * len(w) + r
+    pair = np.unique(pair[np.concatenate([[True], pair[1:] != pair[:-1]])])
+    off = np.searchsorted(pair, np.arange(n + 1) * len(w))
+    return off.astype(np.int32), (pair % len(w)).astype(np.int32)
 
 
 # Workgroups a cooperative launch aims for: an item's primitive quartets are
@@ -744,8 +782,8 @@ class FockBuilder:
             L.coop = self._coop(L)
             if L.coop is None or L.precision == MIXED:   # else no launch reads the per-lane lists
                 self.per_lane(L)
-            if self.mixed and L.precision == MIXED:
-                self._tier_setup(L)
+        if self.mixed:
+            self._tiers_setup([L for L in self.launches if L.precision == MIXED])
         # per system: shell offsets/sizes, Dsh and F (views of flat buffers)
         self.shell_ao, self.shell_size = [], []
         n_ao = [b.n_ao for b, _ in self.systems]
@@ -789,19 +827,43 @@ class FockBuilder:
         most = int((L.bra.deg[work[:, 0]] * (deg[work[:, 3]] - deg[work[:, 1]])).max())
         parts = max(1, min(COOP_GROUPS // len(work), -(-most // 256), 64))
         c = CoopItems(work, kets, parent, parts)
-        c.dev = tuple(native.to_dev(x) for x in (work, kets, parent))
+        c.dev = tuple(native.to_dev(x) for x in (work, kets, np.arange(len(work), dtype=np.int32)))
+        if L.precision == MIXED:
+            c.cover = coop_cover(L.work, L.ket_list, (work, kets, parent))
         return c
 
+    def _tiers_setup(self, mixed) -> None:
+        """The mixed launches' per-build tiers on the device, initially the
+        plan's: one array of every planned item's, one of every cooperative
+        item's (FP32 where all the planned items under it are)."""
+        plan = [(np.arange(len(L.work)) >= L.n_fp64).astype(np.int32) for L in mixed]
+        flat = native.to_dev(np.concatenate(plan)) if plan else None
+        at = np.concatenate([[0], np.cumsum([len(p) for p in plan])]).astype(np.int64)
+        off, idx, tier, n = [], [], [], 0
+        for L, p, lo, hi in zip(mixed, plan, at, at[1:]):
+            L.tier_dev = flat[lo:hi]
+            self._tier_setup(L)
+            if L.coop is not None:
+                o, i = L.coop.cover
+                off.append(o[:-1].astype(np.int64) + n)
+                idx.append(i.astype(np.int64) + lo)
+                tier.append(np.minimum.reduceat(p[i], o[:-1]))
+                n += len(i)
+        self._cover = None
+        if off:
+            start = np.concatenate([[0], np.cumsum([len(x) for x in tier])])
+            out = native.to_dev(np.concatenate(tier))
+            for L, lo, hi in zip([L for L in mixed if L.coop is not None], start, start[1:]):
+                L.coop.tier = out[lo:hi]
+            self._cover = (native.to_dev(np.concatenate([*off, [n]]).astype(np.int32)),
+                           native.to_dev(np.concatenate(idx).astype(np.int32)), flat, out)
+
     def _tier_setup(self, L: "Launch") -> None:
-        """The device side of a mixed launch's per-build tier choice: the
-        tier array (initially the plan's), and the fj_tier_select record:
-        the bound rule's parameters and, with a learned selector, every work
+        """The device side of a mixed launch's per-build tier choice, its
+        fj_tier_select record: the bound rule's parameters and, with a learned selector, every work
         item's density-free features, standardised, and whether they lie in
         the network's training range."""
         n = L.work.shape[0]
-        plan = np.zeros(n, dtype=np.int32)
-        plan[L.n_fp64:] = 1
-        L.tier_dev = native.to_dev(plan)
         sel = native.FjTierSel()
         sel.work, sel.ket_list = L.work_dev.data_ptr(), L.ket_list_dev.data_ptr()
         sel.n_items, sel.diag, sel.tau = n, int(L.diag), self.tau
@@ -873,8 +935,7 @@ class FockBuilder:
         if L.coop is not None:
             c = L.coop
             native.call_fc(L.cls, c.parts, L.bra.side, L.ket.side, c.dev[0], c.work.shape[0], c.dev[1],
-                           c.dev[2], L.tier_dev if L.precision == MIXED else None, sys, L.diag,
-                           self.tau, stream, self.weights)
+                           c.dev[2], c.tier, sys, L.diag, self.tau, stream, self.weights)
             return
         if L.precision == MIXED:
             native.call_fxm(L.cls, L.threads, L.bra.side, L.ket.side, L.work_dev, L.work.shape[0],
@@ -929,6 +990,8 @@ class FockBuilder:
             jobs = self._tier_jobs()
             if jobs is not None:
                 native.tier_select_jobs(jobs[0], jobs[1], jobs[2], sys, jobs[3], main)
+                if self._cover is not None:
+                    native.tier_cover(*self._cover, main)
         self._built = True
         if n_streams <= 1:
             ws = self._workspace(0)
@@ -1025,6 +1088,12 @@ class FockBuilder:
         for L in self.launches:
             q = self.item_quartets(L)
             if L.precision == MIXED:
+                if L.coop is not None and getattr(self, "_built", False):
+                    c = L.coop
+                    n = (c.work[:, 3] - c.work[:, 1]) * (q[c.parent] > 0)
+                    f32 += int(n[c.tier.cpu().numpy() == 1].sum())
+                    tot += int(n.sum())
+                    continue
                 if L.tier_dev is not None and getattr(self, "_built", False):
                     t = L.tier_dev.cpu().numpy()
                 else:

@@ -218,6 +218,15 @@ def tier_select_jobs(jobs_dev, n_jobs: int, n_items: int, sys, net=None, stream=
              C.c_void_p(ptr(net.P) if net is not None else None)), "fj_tier_select_jobs")
 
 
+def tier_cover(off, items, tier, out, stream=None) -> None:
+    """out[i] = 1 where tier is 1 for all of items[off[i] .. off[i + 1])
+    (fj_tier_cover; device int32 arrays, off one longer than out)."""
+    fn = lib().fj_tier_cover
+    fn.restype = C.c_int
+    check(fn(C.c_void_p(stream_handle(stream)), C.c_int(out.numel()), C.c_void_p(ptr(off)),
+             C.c_void_p(ptr(items)), C.c_void_p(ptr(tier)), C.c_void_p(ptr(out))), "fj_tier_cover")
+
+
 def tier_select(bra: FjSide, ket: FjSide, sys, sel: FjTierSel, stream=None) -> None:
     """The per-build tiers of one mixed launch, on the device (fj_tier_select)."""
     fn = lib().fj_tier_select

@@ -1533,6 +1533,10 @@ typedef struct FjTierJob {
 } FjTierJob;
 int fj_tier_select_jobs(fj_stream_t stream, int n_jobs, const FjTierJob* jobs, int n_items,
                         const FjSys* sys, int n_feat, const unsigned short* Wb, const float* P);
+/* The tiers of cooperative items (fj_fc_) from those of the planned items
+ * under them: out[i] = 1 (FP32) where tier[items[e]] is 1 for every e of
+ * [off[i], off[i + 1]), i < n.  Device arrays. */
+int fj_tier_cover(fj_stream_t stream, int n, const int* off, const int* items, const int* tier, int* out);
 
 /* The split HGP J and K kernels (upstream eri/hjk/kernel_hj.py:1-140 and
  * kernel_hk.py:1-110, canonical class mode; parameter list params_of,

@@ -100,3 +100,25 @@ def test_cooperative_items_are_the_plan(kw, batch):
             assert 0 < k1 - k0 <= batch and L.work[p][0] == b and z == L.work[p][2] & 0xffff
             got += [(int(b), int(k)) for k in kets[k0:k1]]
         assert len(got) == len(set(got)) and set(got) == planned
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(lane_flops=1e3), dict(lane_flops=3e4), dict(lane_flops=1e30)])
+def test_cooperative_items_know_every_planned_item_under_them(kw):
+    """A quartet's chunks may lie in several planned items, each with a tier
+    of its own: the item that takes the quartet whole names all of them."""
+    fb, _ = _builder(mixed=True, **kw)
+    several = 0
+    for L in fb.launches:
+        items = fock.coop_items(L.work, L.ket_list, 3)
+        off, under = fock.coop_cover(L.work, L.ket_list, items)
+        holds: dict = {}   # (bra, ket) -> planned items with a chunk of it
+        for p, (b, k0, z, k1) in enumerate(L.work):
+            for e in L.ket_list[k0:k1]:
+                holds.setdefault((int(b), int(e) & 0x1ffff), set()).add(p)
+        work, kets, parent = items
+        assert len(off) == len(work) + 1 and off[-1] == len(under)
+        for i, (b, k0, z, k1) in enumerate(work):
+            want = set().union(*(holds[int(b), int(k)] for k in kets[k0:k1]))
+            assert set(under[off[i]:off[i + 1]].tolist()) == want and parent[i] in want
+            several += len(want) > 1
+    assert (several > 0) == (kw != dict(lane_flops=1e30))

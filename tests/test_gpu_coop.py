@@ -59,9 +59,10 @@ def test_cooperative_batch_and_streams():
 
 
 def test_cooperative_tiers_and_replays():
-    """A mixed build in either form: the tiers are the plan's, so both send
-    the same items to FP32 and agree to the FP32 tier's error (2e-11 on this
-    system's size); replays equal the eager build."""
+    """A mixed build in either form: both choose tiers for the plan's items,
+    and the cooperative one keeps in FP64 the quartets that lie in items of
+    both tiers; they agree to the FP32 tier's error (2e-11 on this system's
+    size); replays equal the eager build."""
     _need_gpu()
     from felizjueves_amd import native
     from felizjueves_amd.systems import closed_shell_density, config2
@@ -74,9 +75,44 @@ def test_cooperative_tiers_and_replays():
     for k in range(3):
         Gc = coop.replay()[0]
         assert np.abs((Gc - Gl).cpu().numpy()).max() <= 1e-10
-        assert coop.fp32_share() == lane.fp32_share() > 0
+        assert 0 < coop.fp32_share() <= lane.fp32_share()
         Dd.copy_(native.to_dev(closed_shell_density(rng, s.basis.n_ao, 20 + k)))
         Gl = lane.build([Dd])[0]
+
+
+@pytest.mark.parametrize("lane_flops", [None, 3e4])
+def test_split_quartets_run_in_fp32_only_where_every_chunk_may(lane_flops):
+    """The network judges a planned item by that item's features, so the items
+    of a split quartet may get different tiers: after a build, a cooperative
+    item is in FP32 where all the planned items under it are, and nowhere
+    else; also for tiers set at random, which no launch's items share."""
+    _need_gpu()
+    from pathlib import Path
+    from felizjueves_amd import native
+    from felizjueves_amd.fock import MIXED, FockBuilder
+    from felizjueves_amd.selector import LearnedSelector
+    from felizjueves_amd.systems import config2
+    sel = LearnedSelector.load(Path(__file__).resolve().parent.parent / "felizjueves_amd" / "tuned" / "selector")
+    s = config2(seed=2, n_atoms=10)
+    fb = FockBuilder(s.basis, s.D, tau=1e-12, mixed=True, selector=sel, lane_flops=lane_flops, coop=True)
+    G64 = FockBuilder(s.basis, s.D, tau=1e-12).build(native.to_dev(s.D)).cpu().numpy()
+    G = fb.build(native.to_dev(s.D), n_streams=4).cpu().numpy()
+    assert np.abs(G - G64).max() <= 1e-8 and fb.fp32_share() > 0
+    rng = np.random.default_rng(1)
+    raised = 0
+    for tiers in (None, 0.5, 0.9):
+        if tiers is not None:
+            flat = fb._cover[2]
+            flat.copy_(native.to_dev((rng.random(flat.numel()) < tiers).astype(np.int32)))
+            native.tier_cover(*fb._cover)
+        for L in fb.launches:
+            assert L.precision == MIXED and L.coop is not None
+            t, got = L.tier_dev.cpu().numpy(), L.coop.tier.cpu().numpy()
+            off, under = L.coop.cover
+            want = np.array([t[under[a:b]].min() for a, b in zip(off, off[1:])])
+            assert np.array_equal(got, want)
+            raised += int((t[L.coop.parent] > got).sum())
+    assert raised > 0
 
 
 def test_cooperative_entry_refuses():
