@@ -359,7 +359,9 @@ class FockBuilder:
     independent systems in the same launches: every class pair of every
     system is one launch per tier, each work item naming its system."""
 
-    weights = (2.0, -0.5)   # of the Coulomb and exchange blocks: J - K/2 (hjk.HJKBuild takes J or K)
+    # of the Coulomb and exchange blocks: J - K/2. Others (hjk.HJKBuild: J or K)
+    # in the cooperative form alone; `launch` refuses them in any other.
+    weights = (2.0, -0.5)
 
     def __init__(self, basis: Basis, D: np.ndarray, *, tau: float = 1e-12, threads=64,
                  mixed: bool = False, fp32_error: float = 1e-11, selector=None,
@@ -937,6 +939,9 @@ class FockBuilder:
             native.call_fc(L.cls, c.parts, L.bra.side, L.ket.side, c.dev[0], c.work.shape[0], c.dev[1],
                            c.dev[2], c.tier, sys, L.diag, self.tau, stream, self.weights)
             return
+        if tuple(self.weights) != FockBuilder.weights:
+            raise ValueError(f"weights {tuple(self.weights)}: the launch of class pair {L.cls} is not cooperative, "
+                             f"and the other kernels build J - K/2 alone")
         if L.precision == MIXED:
             native.call_fxm(L.cls, L.threads, L.bra.side, L.ket.side, L.work_dev, L.work.shape[0],
                             L.n_fp64, sys, L.diag, self.tau, stream, L.ket_list_dev, ws,

@@ -152,3 +152,25 @@ def test_refusals():
         hjk.hjk_launches(co.basis, co.density, tau=1e-12)
     with pytest.raises(ValueError):
         hjk.hjk_launches(fx.basis, fx.density, tau=1e-12, prim_chunk=-1)
+
+
+@pytest.mark.parametrize("precision", [0, 2])
+def test_a_launch_without_the_cooperative_form_refuses_other_weights(precision, monkeypatch):
+    """The per-lane and f-class kernels digest J - K/2: a builder of J or K
+    alone gets an error from such a launch, not their result."""
+    from felizjueves_amd import fock, native
+    fx = load_fixture("h2o_631g")
+    fb = fock.FockBuilder(fx.basis, fx.density, planner="python")
+    ran = []
+    monkeypatch.setattr(native, "call_fx", lambda *a, **k: ran.append("fx"))
+    monkeypatch.setattr(native, "call_fxm", lambda *a, **k: ran.append("fxm"))
+    L = fb.launches[0]
+    L.precision = precision
+    for w in ((2.0, 0.0), (0.0, 1.0)):
+        fb.weights = w
+        with pytest.raises(ValueError, match="J - K/2 alone"):
+            fb.launch(L, None)
+    assert not ran
+    fb.weights = (2.0, -0.5)
+    fb.launch(L, None)
+    assert ran == ["fx" if precision == 0 else "fxm"]
