@@ -92,6 +92,10 @@ KET_INDEX_LIMIT = 1 << 17  # ket-list entries: pair index in bits 0-16
 SELECTOR_PLAN_PAIRS = 50_000
 
 
+class KetIndexError(ValueError):
+    """A class has more shell pairs than a ket-list entry can name."""
+
+
 @dataclass
 class SideTable:
     cls: tuple
@@ -463,8 +467,8 @@ class FockBuilder:
         self.tables = {}
         for c, mps in sorted(by_cls.items()):
             if len(mps) >= KET_INDEX_LIMIT:
-                raise ValueError(f"{len(mps)} shell pairs of class {c}: a ket-list entry holds "
-                                 f"pair indices below {KET_INDEX_LIMIT}")
+                raise KetIndexError(f"{len(mps)} shell pairs of class {c}: a ket-list entry holds "
+                                    f"pair indices below {KET_INDEX_LIMIT}")
             mps = sorted(mps, key=lambda mp: (mp[0], -mp[1].degree, -mp[1].G))
             ps = [p for _, p in mps]
             mol = np.array([m for m, _ in mps], dtype=np.int64)

@@ -392,13 +392,13 @@ class HJKBuild:
         self.builder = None
         # (a width the split kernels refuse goes to them)
         if plan is None and (threads <= 0 or (threads % 64 == 0 and threads <= 256)):
-            from .fock import FockBuilder
+            from .fock import FockBuilder, KetIndexError
             # the fused screen tests G_ab G_cd max(2 D_ab, 2 D_cd, D_ac / 2, ..): at
             # tau / 2 max|D| it and the density-free one pass what the split one does
             t = float(tau) / (2.0 * max(1.0, float(np.abs(D).max())))
             try:
                 self.builder = FockBuilder(basis, D, tau=t, coop=True)
-            except ValueError:   # a class of more pairs than a ket list can name
+            except KetIndexError:   # the split kernels take any number of pairs
                 self._stage(D)
                 return
             self.builder.weights = (2.0, 0.0) if screen == "j" else (0.0, 1.0)

@@ -174,3 +174,22 @@ def test_a_launch_without_the_cooperative_form_refuses_other_weights(precision, 
     fb.weights = (2.0, -0.5)
     fb.launch(L, None)
     assert ran == ["fx" if precision == 0 else "fxm"]
+
+
+def test_split_build_hides_no_refusal_of_the_builder(monkeypatch):
+    """Without a plan the build goes to the split kernels only where a class
+    has more pairs than a ket list names; any other refusal is the caller's."""
+    from felizjueves_amd import fock
+    fx = load_fixture("h2o_sto3g")
+    staged = []
+    monkeypatch.setattr(hjk.HJKBuild, "_stage", lambda self, D: staged.append(self.plan))
+    monkeypatch.setattr(fock, "KET_INDEX_LIMIT", 5)
+    b = hjk.HJKBuild(fx.basis, fx.density)
+    assert staged == [b.plan] and b.builder is None
+
+    def refuse(*a, **k):
+        raise ValueError("refused")
+    monkeypatch.setattr(fock.FockBuilder, "_setup", refuse)
+    with pytest.raises(ValueError, match="refused"):
+        hjk.HJKBuild(fx.basis, fx.density)
+    assert len(staged) == 1
