@@ -193,3 +193,19 @@ def test_split_build_hides_no_refusal_of_the_builder(monkeypatch):
     with pytest.raises(ValueError, match="refused"):
         hjk.HJKBuild(fx.basis, fx.density)
     assert len(staged) == 1
+
+
+def test_split_build_counts_what_it_runs(monkeypatch):
+    """The unique quartets of the builder's plan without a plan given, every
+    ordered one with (no screen drops any at tau = 0)."""
+    from felizjueves_amd import fock, native
+    fx = load_fixture("h2o_sto3g")
+    monkeypatch.setattr(fock.FockBuilder, "to_device", lambda self: setattr(self, "F", None))
+    monkeypatch.setattr(native, "to_dev", lambda x: x)
+    n = fx.basis.n_sh
+    b = hjk.HJKBuild(fx.basis, fx.density, tau=0.0)
+    assert b.quartets_computed == b.builder.n_quartets and b.flops == b.builder.flops > 0
+    assert b.quartets_computed < n ** 4
+    monkeypatch.setattr(hjk, "GpuHJKRunner", lambda: type("R", (), {"zeros": lambda self, n: None})())
+    b = hjk.HJKBuild(fx.basis, fx.density, tau=0.0, plan=hjk.hjk_launches(fx.basis, fx.density, tau=0.0))
+    assert b.quartets_computed == n ** 4 and b.builder is None
