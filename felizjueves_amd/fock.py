@@ -172,33 +172,37 @@ def coop_cover(work: np.ndarray, ket_list: np.ndarray, items):
     list, parent): every planned item that holds some chunk of an item's
     quartets. The error rule clears a planned item's chunks for FP32, so an
     item may run in FP32 only where all of these may."""
-    cw, ck, parent = items
-    n = len(cw)
-    w = work.astype(np.int64)
-    if not (ket_list >> 17).any() and not (w[:, 2] >> 16).any():   # no quartet is split
-        return np.arange(n + 1, dtype=np.int32), parent.astype(np.int32)
-
-    def entries(lo, hi):   # (range, entry) of the entries of the ranges [lo, hi)
-        r = np.repeat(np.arange(len(lo)), hi - lo)
-        return r, np.arange(len(r)) + np.repeat(lo - (np.cumsum(hi - lo) - (hi - lo)), hi - lo)
-    # each list entry's cooperative item: first chunks by their place, later
-    # ones by their quartet (bra, ket), among the first chunks of split kets
-    first = np.nonzero((ket_list & (0x7f << 17)) == 0)[0]
-    later = np.nonzero(ket_list & (0x7f << 17))[0]
-    r, at = entries(cw[:, 1].astype(np.int64), cw[:, 3].astype(np.int64))
-    of = np.empty(len(ket_list), dtype=np.int64)
-    of[first[at]] = r
-    whole_bra = np.nonzero(((w[:, 2] >> 16) & 0xff) == 0)[0]
-    r, at = entries(w[whole_bra, 1], w[whole_bra, 3])
-    quartet = np.empty(len(ket_list), dtype=np.int64)
-    quartet[at] = w[whole_bra[r], 0] << 17
-    quartet |= ket_list & 0x1ffff
-    split = first[ket_list[first] >> 24 != 0]
-    split = split[np.argsort(quartet[split])]
-    of[later] = of[split[np.searchsorted(quartet[split], quartet[later])]]
-    r, at = entries(w[:, 1], w[:, 3])
-    pair = of[at] * len(w) + r
-    pair = np.unique(pair[np.concatenate([[True], pair[1:] != pair[:-1]])])
+    cw, _, parent = items
+    n, w = len(cw), work.astype(np.int64)
+    pairs = [np.arange(n) * len(w) + parent]   # (item, planned item); whole quartets have no other
+    chunk0 = np.nonzero(((w[:, 2] >> 16) & 0xff) == 0)[0]
+    chunked = np.nonzero(w[:, 2] >> 16)[0]     # a range of the bra's primitives
+    lo = (ket_list >> 17) & 0x7f
+    cut = np.nonzero(ket_list >> 17)[0]        # lanes with a range of the ket's
+    if len(cut) or len(chunked):
+        # the planned item (of the first bra chunk) and the item of an entry
+        by_start = chunk0[np.argsort(w[chunk0, 1])]
+        by_first = np.argsort(cw[:, 1])
+        at = np.cumsum(lo == 0) - 1
+        under = lambda e: by_start[np.searchsorted(w[by_start, 1], e, side="right") - 1]       # noqa: E731
+        of_first = lambda e: by_first[np.searchsorted(cw[by_first, 1], at[e], side="right") - 1]   # noqa: E731
+        plan = under(cut)
+        # a later chunk is found by its quartet (bra, ket) among the cut first ones
+        quartet = (w[plan, 0] << 17) | (ket_list[cut] & 0x1ffff)
+        f = np.nonzero(lo[cut] == 0)[0]
+        f = f[np.argsort(quartet[f])]
+        of = of_first(cut[f])[np.searchsorted(quartet[f], quartet)]
+        pairs.append(of * len(w) + plan)
+        if len(chunked):   # their lists are their first chunk's: every lane of it
+            full = np.empty(len(ket_list), dtype=np.int64)
+            first = np.nonzero(lo == 0)[0]
+            full[first] = of_first(first)
+            full[cut] = of
+            m = w[chunked, 3] - w[chunked, 1]
+            r = np.repeat(np.arange(len(chunked)), m)
+            e = np.arange(len(r)) + np.repeat(w[chunked, 1] - (np.cumsum(m) - m), m)
+            pairs.append(full[e] * len(w) + chunked[r])
+    pair = np.unique(np.concatenate(pairs))
     off = np.searchsorted(pair, np.arange(n + 1) * len(w))
     return off.astype(np.int32), (pair % len(w)).astype(np.int32)
 
