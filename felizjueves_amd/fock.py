@@ -213,6 +213,25 @@ def coop_cover(work: np.ndarray, ket_list: np.ndarray, items):
 COOP_GROUPS = 1024
 
 
+# Quartets of a launch from which the per-lane form is the faster one, for the
+# class pairs where it is on a full chip (by more than 7%; the cooperative
+# form stays the faster one, or within that, everywhere else): where the two
+# forms' times of the default plan's launches cross, between clusters of 28 to
+# 80 atoms s,s,p,d and a batch of 16 molecules, e.g. (sd|dd), per-lane /
+# cooperative ms: 124 thousand quartets 2.78 / 2.21, 274 thousand 5.33 / 5.89,
+# 2.2 million 27.8 / 37.0; (dd|dd): 84 thousand 11.9 / 9.9, 648 thousand 51.6 /
+# 61.8. Below the line the per-lane form's few long lanes leave the chip idle;
+# above it the lanes are enough, and it pays no LDS sums. Whole builds, four
+# streams, per-lane / cooperative / by this rule: 40 atoms 75.0 / 66.2 / 64.9
+# ms, 64 atoms 214 / 218 / 200 ms, the 16 molecules 1,098 / 1,200 / 1,074 ms.
+PER_LANE_QUARTETS = {
+    (0, 0, 0, 0): 1_900_000, (0, 1, 0, 1): 3_100_000, (0, 2, 0, 2): 930_000, (0, 2, 1, 1): 780_000,
+    (0, 2, 1, 2): 1_300_000, (0, 2, 2, 0): 520_000, (0, 2, 2, 2): 220_000, (1, 1, 1, 1): 620_000,
+    (1, 1, 2, 0): 1_400_000, (1, 2, 2, 2): 195_000, (2, 0, 2, 0): 1_000_000, (2, 1, 2, 2): 390_000,
+    (2, 2, 2, 2): 110_000,
+}
+
+
 WAVE = 64             # lanes of a wavefront
 FILL_MIN_PRIMS = 4    # a lane is halved to fill idle lanes only from this many primitive pairs
 
@@ -414,11 +433,11 @@ class FockBuilder:
         launches. None: every class pair.
         coop: whether a launch runs in the quartet-cooperative form
         (fj_fc_*; classes through d). None: every one, except a class pair
-        whose threads or lane_flops are given (they shape the per-lane
-        form). True / False: every class pair that has it / none. Measured,
+        whose threads or lane_flops are given (they shape the per-lane form)
+        and a launch past its class pair's PER_LANE_QUARTETS. True / False: every class pair that has it / none. Measured,
         one stream / four, per-lane -> cooperative: the three-atom s,s,p,d
         system 26 -> 1.6 / 15.8 -> 0.5 ms, 9 atoms 31 -> 3.1 / 9.6 -> 1.7 ms,
-        40 atoms 104 -> 67 / 75 -> 66 ms."""
+        40 atoms 104 -> 67 / 75 -> 65 ms."""
         self.coop = coop
         self.merge_tiers = bool(merge_tiers)
         self.orient = bool(orient)
@@ -825,7 +844,8 @@ class FockBuilder:
         keeps the per-lane form."""
         batch = native.coop_batch(L.cls)
         shaped = (self.lane_flops is not None or self.threads != 64 or L.cls in self.class_threads
-                  or L.cls in self.class_lane_flops)
+                  or L.cls in self.class_lane_flops
+                  or L.n_quartets >= PER_LANE_QUARTETS.get(L.cls, L.n_quartets + 1))
         if not batch or L.precision == FP32 or self.coop is False or (self.coop is None and shaped):
             return None
         work, kets, parent = coop_items(L.work, L.ket_list, batch)

@@ -122,3 +122,26 @@ def test_cooperative_items_know_every_planned_item_under_them(kw):
             assert set(under[off[i]:off[i + 1]].tolist()) == want and parent[i] in want
             several += len(want) > 1
     assert (several > 0) == (kw != dict(lane_flops=1e30))
+
+
+def test_the_form_of_a_launch(monkeypatch):
+    """A launch past its class pair's PER_LANE_QUARTETS keeps the per-lane form
+    by default; coop says otherwise, and a class pair without a line, or a
+    shaped one, has no such choice."""
+    monkeypatch.setattr(fock.native, "coop_batch", lambda cls: 4)
+    monkeypatch.setattr(fock.native, "to_dev", lambda x: x)
+    fb, _ = _builder()
+    lines = 0
+    for L in fb.launches:
+        line = fock.PER_LANE_QUARTETS.get(L.cls)
+        for n, per_lane in ((1, False), (10 ** 9, line is not None)) + (((line - 1, False), (line, True)) if line else ()):
+            L.n_quartets = n
+            for coop, want in ((None, per_lane), (True, False), (False, True)):
+                fb.coop = coop
+                assert (fb._coop(L) is None) == want, (L.cls, n, coop)
+        lines += line is not None
+        fb.coop, fb.class_threads = None, {L.cls: 64}
+        L.n_quartets = 1
+        assert fb._coop(L) is None
+        fb.class_threads = {}
+    assert lines == len(fock.PER_LANE_QUARTETS)
