@@ -58,6 +58,41 @@ def test_cooperative_batch_and_streams():
         _close(a, b)
 
 
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("form", ["lane", "tuned", "some"])
+def test_per_lane_launches_on_streams_and_in_a_graph(form, mixed):
+    """Per-lane launches, classes with a workspace among them, alone and
+    beside cooperative ones (the shipped 40-atom configuration; a few class
+    pairs named) on four streams, eager and replayed, for two densities,
+    against the oracle at the bars of either tier."""
+    _need_gpu()
+    from felizjueves_amd import autotune, native
+    from felizjueves_amd.fock import FockBuilder
+    from felizjueves_amd.systems import closed_shell_density, config2
+    from test_builder_oracle import oracle_build
+    s = config2(seed=2, n_atoms=10)
+    named = {(2, 2, 2, 2): 128, (0, 2, 2, 2): 64, (1, 1, 1, 2): 256, (0, 0, 0, 0): 64}
+    kw = {"lane": dict(coop=False), "some": dict(threads=named, lane_flops={c: 3e5 for c in named}),
+          "tuned": autotune.builder_kwargs(autotune.load(autotune.Path(autotune.__file__).parent / "tuned" /
+                                                         "c2_40atom.json"))}[form]
+    fb = FockBuilder(s.basis, s.D, tau=1e-12, mixed=mixed, **kw)
+    Dd = native.to_dev(s.D)
+    fb.capture(Dd, n_streams=4)
+    lane = [L for L in fb.launches if L.coop is None]
+    assert any(native.workspace_bytes(L.cls, L.threads, len(L.work)) for L in lane)
+    assert (len(lane) == len(fb.launches)) == (form == "lane")
+    bar = 1e-8 if mixed else 1e-10
+    for D in (s.D, closed_shell_density(np.random.default_rng(3), s.basis.n_ao, 20)):
+        Dd.copy_(native.to_dev(D))
+        Go = oracle_build(FockBuilder(s.basis, D, tau=1e-12), D)
+        worst = 0.0
+        for _ in range(3):
+            worst = max(worst, np.abs(fb.replay().cpu().numpy() - Go).max())
+            worst = max(worst, np.abs(fb.build(Dd, n_streams=4).cpu().numpy() - Go).max())
+        print(form, mixed, "max|dG|", worst, "per-lane", len(lane), "of", len(fb.launches), flush=True)
+        assert worst <= bar
+
+
 def test_cooperative_tiers_and_replays():
     """A mixed build in either form: both choose tiers for the plan's items,
     and the cooperative one keeps in FP64 the quartets that lie in items of
