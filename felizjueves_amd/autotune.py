@@ -1,10 +1,11 @@
-"""Autotuner of the batched Fock build: per class pair, the lanes per work
-item (threads) and the primitive-loop split (lane_flops), then the number
-of streams the launches are dealt to.
+"""Autotuner of the batched Fock build: per class pair, the cooperative form
+or, per lane, the lanes per work item (threads) and the primitive-loop split
+(lane_flops), then the number of streams the launches are dealt to.
 
 Each candidate plan is timed on the device: HIP events around every launch
 of a whole build (median over repeats), summed per class pair over its
-tiers. The fastest candidate per class pair is kept; the tuned plan is then
+tiers. The fastest per-lane candidate per class pair is kept unless the
+cooperative form is over COOP_MARGIN faster; the tuned plan is then
 timed as whole captured builds for each stream count. The choice is a pure
 function of the measured times, written to / read from a JSON file so that
 a tuned configuration can be reused without measuring again.
@@ -24,6 +25,11 @@ from .fock import FockBuilder
 THREADS = (64, 128, 256)
 LANE_FLOPS = (3.0e4, 1.0e5, 3.0e5, 1.0e6)
 STREAMS = (1, 2, 4)
+# A launch that fills the chip gains less from others on other streams than one
+# of few wavefronts, so the cooperative form has to be this much faster alone
+# (40 atoms, production: 70.8 ms with no class pair cooperative, 59.5 with
+# those 10% faster, 66.2 with all).
+COOP_MARGIN = 0.1
 
 
 def launch_times(fb: FockBuilder, D_devs, reps: int = 3) -> dict:
@@ -69,7 +75,9 @@ def build_time(fb: FockBuilder, D_devs, n_streams: int, steps: int = 10) -> floa
 def tune(systems, threads=THREADS, lane_flops=LANE_FLOPS, streams=STREAMS, log=None, **kw) -> dict:
     """Tune the build of `systems` [(basis, D), ...] (other FockBuilder
     keywords in kw). Returns {"threads": {cls: t}, "lane_flops": {cls: lf},
-    "n_streams": s, "ms": {...}} with class pairs as 'labcd' strings."""
+    "coop": [cls], "cooperative_ms": {cls: [best per-lane, cooperative]},
+    "n_streams": s, ...} with class pairs as 'labcd' strings, each in "coop"
+    or in the other two."""
     D_devs = [native.to_dev(D) for _, D in systems]
     best: dict = {}
     table = {}
@@ -84,23 +92,31 @@ def tune(systems, threads=THREADS, lane_flops=LANE_FLOPS, streams=STREAMS, log=N
             if log:
                 log(t, lf, sum(ms.values()))
             del fb
-    th = {c: b[1] for c, b in best.items()}
-    lfs = {c: b[2] for c, b in best.items()}
-    fb = FockBuilder.batch(systems, threads=th, lane_flops=lfs, **kw)
+    fb = FockBuilder.batch(systems, coop=True, **kw)
+    ms = launch_times(fb, D_devs)
+    has = {L.cls for L in fb.launches if L.coop is not None}
+    both = {c: (best[c][0], ms[c]) for c in sorted(has) if c in best}
+    coop = [c for c, (lane, co) in both.items() if co < (1.0 - COOP_MARGIN) * lane]
+    if log:
+        log("cooperative", sum(ms.values()), f"{len(coop)} class pairs")
+    del fb
+    name = lambda c: "".join(map(str, c))  # noqa: E731
+    cfg = {"threads": {name(c): b[1] for c, b in best.items() if c not in coop},
+           "lane_flops": {name(c): b[2] for c, b in best.items() if c not in coop},
+           "coop": [name(c) for c in coop], "cooperative_ms": {name(c): list(v) for c, v in both.items()}}
+    fb = FockBuilder.batch(systems, **builder_kwargs(cfg), **kw)
     st = {s: build_time(fb, D_devs, s) for s in streams}
     n_streams = min(st, key=st.get)
     if log:
         log("streams", st)
-    return {"threads": {"".join(map(str, c)): v for c, v in th.items()},
-            "lane_flops": {"".join(map(str, c)): v for c, v in lfs.items()},
-            "n_streams": n_streams, "graph_ms": {str(k): v for k, v in st.items()},
+    return {**cfg, "n_streams": n_streams, "graph_ms": {str(k): v for k, v in st.items()},
             "launch_ms": table}
 
 
 def tier_pays(systems, tuned: dict, margin: float = 0.02, log=None, **kw) -> list:
     """The class pairs whose mixed launch (per-item FP32 / FP64 tiers, kw
     the mixed builder's keywords, e.g. the selector) is measured faster than
-    their FP64 launch at the tuned threads and split, by more than
+    their FP64 launch in the tuned form, threads and split, by more than
     `margin`: a mixed build sends work to the FP32 tier only there (on
     MI355X, FP32 VALU without packed math issues at the FP64 rate, so the
     tier pays only where its smaller register footprint does)."""
@@ -124,15 +140,13 @@ def load(path: Path) -> dict:
 
 
 def builder_kwargs(cfg: dict) -> dict:
-    """FockBuilder keywords of a tuned configuration. A class pair without an
-    entry runs in the builder's cooperative form: `cooperative_ms`, where a
-    configuration has it, holds each launch's [tuned per-lane, cooperative]
-    times, and class pairs over 10% faster cooperatively have no entry (40
-    atoms, production: 70.8 -> 59.5 ms against every entry kept, 66.2 with
-    none)."""
+    """FockBuilder keywords of a tuned configuration. A class pair with no
+    entry and not in "coop" takes the form of the builder's default rule."""
     key = lambda s: tuple(int(ch) for ch in s)  # noqa: E731
     out = {"threads": {key(k): v for k, v in cfg["threads"].items()},
            "lane_flops": {key(k): v for k, v in cfg["lane_flops"].items()}}
+    if "coop" in cfg:
+        out["coop"] = {key(k) for k in cfg["coop"]}
     return out
 
 
@@ -146,7 +160,7 @@ def mixed_kwargs(cfg: dict) -> dict:
 
 
 def main() -> None:
-    """Tune a workload (--tune: per class pair threads and split, then the
+    """Tune a workload (--tune: per class pair form, threads and split, then the
     stream count) and / or measure where the FP32 tier pays for the tuned
     configuration (`fp32_classes`), writing the configuration file.
 
@@ -161,7 +175,7 @@ def main() -> None:
     ap = argparse.ArgumentParser()
     ap.add_argument("config", help="tuned configuration file (JSON) to update or create")
     ap.add_argument("--workload", choices=("c1", "c2", "c4"), required=True)
-    ap.add_argument("--tune", action="store_true", help="run the threads / split / streams search first")
+    ap.add_argument("--tune", action="store_true", help="run the form / threads / split / streams search first")
     ap.add_argument("--every", type=int, default=4, help="c4: tune on every N-th molecule")
     ap.add_argument("--lane-flops", type=float, nargs="+", default=list(LANE_FLOPS),
                     help="the primitive-loop split candidates (FLOPs per lane)")

@@ -434,11 +434,13 @@ class FockBuilder:
         coop: whether a launch runs in the quartet-cooperative form
         (fj_fc_*; classes through d). None: every one, except a class pair
         whose threads or lane_flops are given (they shape the per-lane form)
-        and a launch past its class pair's PER_LANE_QUARTETS. True / False: every class pair that has it / none. Measured,
+        and a launch past its class pair's PER_LANE_QUARTETS. True / False:
+        every class pair that has it / none. Class pairs (la, lb, lc, ld):
+        these (the autotuner's choice), the others as with None. Measured,
         one stream / four, per-lane -> cooperative: the three-atom s,s,p,d
         system 26 -> 1.6 / 15.8 -> 0.5 ms, 9 atoms 31 -> 3.1 / 9.6 -> 1.7 ms,
         40 atoms 104 -> 67 / 75 -> 65 ms."""
-        self.coop = coop
+        self.coop = coop if coop is None or isinstance(coop, bool) else {tuple(int(x) for x in c) for c in coop}
         self.merge_tiers = bool(merge_tiers)
         self.orient = bool(orient)
         self.fp32_classes = None if fp32_classes is None else {tuple(int(x) for x in c)
@@ -843,10 +845,15 @@ class FockBuilder:
         """The launch's items for the cooperative kernel, or None when it
         keeps the per-lane form."""
         batch = native.coop_batch(L.cls)
-        shaped = (self.lane_flops is not None or self.threads != 64 or L.cls in self.class_threads
-                  or L.cls in self.class_lane_flops
-                  or L.n_quartets >= PER_LANE_QUARTETS.get(L.cls, L.n_quartets + 1))
-        if not batch or L.precision == FP32 or self.coop is False or (self.coop is None and shaped):
+        if isinstance(self.coop, bool):
+            coop = self.coop
+        elif self.coop is not None and L.cls in self.coop:
+            coop = True
+        else:
+            shaped = (self.lane_flops is not None or self.threads != 64 or L.cls in self.class_threads
+                      or L.cls in self.class_lane_flops)
+            coop = not shaped and L.n_quartets < PER_LANE_QUARTETS.get(L.cls, L.n_quartets + 1)
+        if not batch or L.precision == FP32 or not coop:
             return None
         work, kets, parent = coop_items(L.work, L.ket_list, batch)
         if not len(work):

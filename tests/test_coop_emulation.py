@@ -136,7 +136,7 @@ def test_the_form_of_a_launch(monkeypatch):
         line = fock.PER_LANE_QUARTETS.get(L.cls)
         for n, per_lane in ((1, False), (10 ** 9, line is not None)) + (((line - 1, False), (line, True)) if line else ()):
             L.n_quartets = n
-            for coop, want in ((None, per_lane), (True, False), (False, True)):
+            for coop, want in ((None, per_lane), (True, False), (False, True), ({L.cls}, False), (set(), per_lane)):
                 fb.coop = coop
                 assert (fb._coop(L) is None) == want, (L.cls, n, coop)
         lines += line is not None
@@ -145,3 +145,31 @@ def test_the_form_of_a_launch(monkeypatch):
         assert fb._coop(L) is None
         fb.class_threads = {}
     assert lines == len(fock.PER_LANE_QUARTETS)
+
+
+def test_the_tuner_chooses_between_the_forms(monkeypatch):
+    """A class pair over COOP_MARGIN faster cooperatively than in its best
+    per-lane shape is tuned to that form, any other to its shape, and the
+    configuration builds so whatever the default rule says."""
+    from felizjueves_amd import autotune
+    monkeypatch.setattr(fock.native, "coop_batch", lambda cls: 4)
+    monkeypatch.setattr(fock.native, "to_dev", lambda x: x)
+    monkeypatch.setattr(fock, "PER_LANE_QUARTETS", {(0, 0, 0, 0): 1})
+    fb, D = _builder()
+
+    def launch_times(fb, D_devs, reps=3):   # (pp|dd) cooperatively 1% faster than the best shape, the rest 20%
+        for L in fb.launches:
+            L.coop = fb._coop(L)
+        return {L.cls: (0.99 if L.cls == (1, 1, 2, 2) else 0.8) if L.coop is not None
+                else 1.0 + abs(L.threads - 128) / 64 for L in fb.launches}
+    monkeypatch.setattr(autotune, "launch_times", launch_times)
+    monkeypatch.setattr(autotune, "build_time", lambda fb, D_devs, n, steps=10: float(n))
+    cfg = autotune.tune([(fb.basis, D)], planner="python")
+    assert cfg["threads"] == {"1122": 128} and set(cfg["lane_flops"]) == {"1122"} and cfg["n_streams"] == 1
+    assert cfg["cooperative_ms"]["1122"] == [1.0, 0.99] and cfg["cooperative_ms"]["0000"] == [1.0, 0.8]
+    assert len(cfg["coop"]) == len(fb.launches) - 1
+    tuned = fock.FockBuilder(fb.basis, D, planner="python", **autotune.builder_kwargs(cfg))
+    assert {L.cls for L in tuned.launches if tuned._coop(L) is None} == {(1, 1, 2, 2)}
+    cfg.pop("coop")   # an older configuration: the default rule
+    old = fock.FockBuilder(fb.basis, D, planner="python", **autotune.builder_kwargs(cfg))
+    assert {L.cls for L in old.launches if old._coop(L) is None} == {(1, 1, 2, 2), (0, 0, 0, 0)}
