@@ -1,5 +1,6 @@
-// Emulate the quartet-cooperative F kernel of one class (gen/c_<cls>.h) on
-// the CPU over a builder work list read from a binary file; writes F.
+// Emulate an F kernel of one class over a builder work list read from a
+// binary file; writes F: the quartet-cooperative one (gen/c_<cls>.h), or the
+// call CALL of any other, with GRID_Z workgroups to each (x, y).
 // 256 threads, one per lane, one workgroup at a time. TEST INFRASTRUCTURE.
 #include "fj_device.h"   // the emulation header, copied under this name
 #include <fstream>
@@ -14,6 +15,10 @@ thread_local int g_mf_parity;
 double g_shfl[256];
 double* g_dyn_lds;
 #include CLS_HEADER
+#ifndef CALL
+#define CALL KERNEL<true>(a, parent, 2.0, -0.5)
+#define GRID_Z 1
+#endif
 
 template <typename T> T* rd(std::ifstream& f) {
     long long n;
@@ -49,18 +54,19 @@ int main(int argc, char** argv) {
     g_bar = &bar;
     g_wbar[0] = &w0; g_wbar[1] = &w1; g_wbar[2] = &w2; g_wbar[3] = &w3;
     blockDim = {256, 1, 1};
-    gridDim = {(unsigned)h[2], (unsigned)h[3], 1};
+    gridDim = {(unsigned)h[2], (unsigned)h[3], GRID_Z};
     std::vector<std::thread> ts;
     for (unsigned t = 0; t < 256; ++t)
         ts.emplace_back([&, t] {
             threadIdx = {t, 0, 0};
-            for (unsigned y = 0; y < gridDim.y; ++y)
-                for (unsigned x = 0; x < gridDim.x; ++x) {
-                    if (t == 0) blockIdx = {x, y, 0};
-                    bar.arrive_and_wait();
-                    KERNEL<true>(a, parent, 2.0, -0.5);
-                    bar.arrive_and_wait();
-                }
+            for (unsigned z = 0; z < gridDim.z; ++z)
+                for (unsigned y = 0; y < gridDim.y; ++y)
+                    for (unsigned x = 0; x < gridDim.x; ++x) {
+                        if (t == 0) blockIdx = {x, y, z};
+                        bar.arrive_and_wait();
+                        CALL;
+                        bar.arrive_and_wait();
+                    }
         });
     for (auto& t : ts) t.join();
     std::ofstream o(argv[2], std::ios::binary);

@@ -31,20 +31,58 @@ def _builder(**kw):
 # one class with each boundary: no HRR, one side's, both; Boys columns from
 # the global table and in LDS; one and several VRR groups; lanes shared over
 # two workgroups; batches of two kets (a batch edge within an item); a batch
-# of every ket of the class
-CASES = [((0, 0, 0, 0), 1, 32), ((0, 1, 0, 1), 2, 2), ((1, 0, 1, 1), 1, 3), ((0, 2, 1, 2), 1, 2), ((0, 1, 2, 2), 2, 32)]
+# of every ket of the class; and (batch None) the plan's own items, which hold
+# chunks of the bra's and of the kets' primitives
+CASES = [((0, 0, 0, 0), 1, 32), ((0, 1, 0, 1), 2, 2), ((1, 0, 1, 1), 1, 3), ((0, 2, 1, 2), 1, 2), ((0, 1, 2, 2), 2, 32),
+         ((0, 1, 1, 1), 2, None)]
+
+
+def run_work_list(fb, D, L, work, kets, parent, parts, tmp_path, flags):
+    """F of launch L's class from the emulated kernel over a work list, and
+    from the oracle's launch of the same tables."""
+    b = fb.basis
+    host = builder_tables_host(fb)
+    Dsh = P.density_blocks(b, D)
+    exe = tmp_path / "emu"
+    r = subprocess.run(["g++", "-std=c++20", "-O1", "-g0", "-fsanitize=address", f"-I{ROOT / 'include'}", f"-I{tmp_path}",
+                        *flags, str(EMU / "coop_emu.cpp"), "-o", str(exe), "-lpthread"], cwd=tmp_path,
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    with open(tmp_path / "case.bin", "wb") as f:
+        np.array([L.bra.n, L.ket.n, len(work), parts, b.n_sh, b.n_ao, L.diag], dtype=np.int32).tofile(f)
+        np.array([fb.tau]).tofile(f)
+
+        def put(x, dt):
+            x = np.ascontiguousarray(x, dtype=dt).ravel()
+            np.array([x.size], dtype=np.int64).tofile(f)
+            x.tofile(f)
+        for c in (L.cls[:2], L.cls[2:]):
+            t = host[c]
+            for k, dt in (("prim", "f8"), ("off", "i4"), ("sep", "f8"), ("G", "f8"), ("sh", "i4"), ("ao", "i4")):
+                put(t[k], dt)
+        for x, dt in ((work, "i4"), (kets, "i4"), (parent, "i4"), (np.zeros(len(L.work)), "i4"), (Dsh, "f8"), (D, "f8")):
+            put(x, dt)
+    r = subprocess.run([str(exe), str(tmp_path / "case.bin"), str(tmp_path / "F.bin")], cwd=tmp_path,
+                       env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"), capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-3000:]
+    F = np.fromfile(tmp_path / "F.bin").reshape(b.n_ao, b.n_ao)
+    Fo = np.zeros_like(F)
+    O.fx_launch(L.cls, host[L.cls[:2]], host[L.cls[2:]], L.diag, b.n_sh, b.n_ao, fb.tau, Dsh, D, Fo, pre=True)
+    assert np.abs(Fo).max() > 0
+    return F, Fo
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
 @pytest.mark.parametrize("cls,parts,batch", CASES)
 def test_cooperative_kernel_on_cpu_vs_oracle(cls, parts, batch, tmp_path):
-    fb, D = _builder()
-    b = fb.basis
+    fb, D = _builder(**(dict(lane_flops=1e3) if batch is None else {}))
     L = [x for x in fb.launches if x.cls == cls][0]
     # items of up to 64 kets, so that the kernel takes several batches per item
-    work, kets, parent = fock.coop_items(L.work, L.ket_list, 64 if batch == 2 else batch)
-    host = builder_tables_host(fb)
-    Dsh = P.density_blocks(b, D)
+    if batch is None:
+        work, kets, parent = L.work, L.ket_list, np.arange(len(L.work))
+        assert (work[:, 2] >> 16).any() and (kets >> 17).any()
+    else:
+        work, kets, parent = fock.coop_items(L.work, L.ket_list, 64 if batch == 2 else batch)
     name = "".join(map(str, cls))
     gen_hip.generate([], tmp_path / "gen")
     gen_hip.generate_coop([cls], tmp_path / "gen")
@@ -56,33 +94,10 @@ def test_cooperative_kernel_on_cpu_vs_oracle(cls, parts, batch, tmp_path):
         h.write_text(t.replace(f"min({n}, (w.w - first", "min(2, (w.w - first").replace(f"first += step * {n})", "first += step * 2)"))
     shutil.copy(EMU / "fj_device_emu.h", tmp_path / "fj_device.h")
     shutil.copy(ROOT / "felizjueves_amd" / "csrc" / "fj_coop.h", tmp_path / "fj_coop.h")
-    exe = tmp_path / "emu"
-    subprocess.run(["g++", "-std=c++20", "-O1", "-g0", "-fsanitize=address", f"-I{ROOT / 'include'}", f"-I{tmp_path}",
-                    f'-DCLS_HEADER="gen/c_{name}.h"', f"-DKERNEL=fj_c_{name}_k", str(EMU / "coop_emu.cpp"),
-                    "-o", str(exe), "-lpthread"], check=True, cwd=tmp_path, capture_output=True)
-    with open(tmp_path / "case.bin", "wb") as f:
-        np.array([L.bra.n, L.ket.n, len(work), parts, b.n_sh, b.n_ao, L.diag], dtype=np.int32).tofile(f)
-        np.array([fb.tau]).tofile(f)
-
-        def put(x, dt):
-            x = np.ascontiguousarray(x, dtype=dt).ravel()
-            np.array([x.size], dtype=np.int64).tofile(f)
-            x.tofile(f)
-        for c in (cls[:2], cls[2:]):
-            t = host[c]
-            for k, dt in (("prim", "f8"), ("off", "i4"), ("sep", "f8"), ("G", "f8"), ("sh", "i4"), ("ao", "i4")):
-                put(t[k], dt)
-        for x, dt in ((work, "i4"), (kets, "i4"), (parent, "i4"), (np.zeros(len(L.work)), "i4"), (Dsh, "f8"), (D, "f8")):
-            put(x, dt)
-    r = subprocess.run([str(exe), str(tmp_path / "case.bin"), str(tmp_path / "F.bin")], cwd=tmp_path,
-                       env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"), capture_output=True, text=True, timeout=600)
-    assert r.returncode == 0, r.stderr[-3000:]
-    F = np.fromfile(tmp_path / "F.bin").reshape(b.n_ao, b.n_ao)
-    Fo = np.zeros_like(F)
-    O.fx_launch(cls, host[cls[:2]], host[cls[2:]], L.diag, b.n_sh, b.n_ao, fb.tau, Dsh, D, Fo, pre=True)
+    F, Fo = run_work_list(fb, D, L, work, kets, parent, parts, tmp_path,
+                          [f'-DCLS_HEADER="gen/c_{name}.h"', f"-DKERNEL=fj_c_{name}_k"])
     # the same recurrences, summed over primitives in another order
     assert np.abs(F - Fo).max() <= 1e-12 * max(1.0, np.abs(Fo).max())
-    assert np.abs(Fo).max() > 0
 
 
 @pytest.mark.parametrize("kw", [dict(), dict(lane_flops=1e3), dict(lane_flops=1e30), dict(mixed=True)])
