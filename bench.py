@@ -98,6 +98,14 @@ def launch_times(fb, Dd, reps=1):
     return out
 
 
+def kernel_name(L) -> str:
+    """The kernel that a builder's FP64 launch runs."""
+    n = "".join(map(str, L.cls))
+    if L.coop is not None:
+        return f"fj_c_{n}_k<false>"
+    return f"fj_fquad_k<{', '.join(map(str, L.cls))}>" if max(L.cls) > 2 else f"fj_f_{n}_k<double>"
+
+
 def load_tuning(name, mixed: bool = False):
     """(builder keywords, stream count) of a tuned configuration; with
     `mixed`, also the class pairs where the FP32 tier was measured to pay."""
@@ -186,8 +194,8 @@ def gradient_block(steps: int, cpu: bool = True) -> dict:
     """The fused two-electron gradient (gradient.py, fj_gf_jobs: one merged
     launch per class) on the three-atom s,s,p,d system and the 10-atom
     cluster. Per system: seconds per gradient (HIP events on the stream
-    the launches go to, around whole gradients), the loop form's FLOPs
-    (gradient.flops) over that time against the FP64 peak, primitive
+    the launches go to, around whole gradients), the matrix-core kernel's
+    FLOPs (gradient.flops) over that time against the FP64 peak, primitive
     quartets/s; on the three-atom system max|dG| against the oracle
     (oracle_grad_ordered) and, unless `cpu` is off, the oracle's time (the
     whole gradient on the host cores)."""
@@ -217,10 +225,10 @@ def gradient_block(steps: int, cpu: bool = True) -> dict:
              "prim_quartets": GR.prim_quartets(st), "classes": len(run.classes),
              "stream_launches": len(st.launches), "seconds_per_gradient": t,
              "gradients_per_s": 1.0 / t, "prim_quartets_per_s": GR.prim_quartets(st) / t,
-             "roofline": {"bound": "fp64_valu", "achieved": fl / t / 1e12, "peak": FP64_PEAK_TFLOPS,
+             "roofline": {"bound": "fp64", "achieved": fl / t / 1e12, "peak": FP64_PEAK_TFLOPS,
                           "unit": "TFLOP/s", "frac": fl / t / 1e12 / FP64_PEAK_TFLOPS,
                           "gflop_per_gradient": fl / 1e9,
-                          "kernel": "fj_gfjobs_k (every class; its launches back to back)"}}
+                          "kernel": "fj_gfquad_k (every class; its launches back to back)"}}
         if key == "c1_3atom":
             G = run.G.cpu().numpy()
             sys.path.insert(0, str(ROOT / "tests"))
@@ -241,14 +249,15 @@ def gradient_block(steps: int, cpu: bool = True) -> dict:
 
 
 def split_jk_block(cpu: bool = True, cluster: bool = True) -> dict:
-    """The split HGP J and K kernels (hjk.py: one kernel per orbit
-    representative, every ordered quartet of the canonical stream, the
-    upstream's split design) on the three-atom system and the 10-atom
-    cluster: ms per J and per K build (hjk.HJKBuild: the launch arguments
-    staged on the device beforehand, spread over hjk.STREAMS streams; HIP
-    events around three replays of the build captured as one HIP graph, and
-    around three eager builds; the faster is the build's time), the
-    quartets passing the in-kernel screen and their algorithmic FLOPs
+    """Split J and K builds (hjk.HJKBuild) on the three-atom system and the
+    10-atom cluster, in both forms: "default", without a plan (the unique
+    quartets through the cooperative kernels), and with a plan (the split
+    kernels, one per orbit representative, every ordered quartet of the
+    canonical stream, the upstream's design). Per form ms per J and per K
+    build (everything staged on the device beforehand, spread over
+    hjk.STREAMS streams; HIP events around three replays of the build
+    captured as one HIP graph, and around three eager builds; the faster is
+    the build's time), the quartets it computes and their algorithmic FLOPs
     (hgp.cost of the kernel's class: VRR per primitive quartet, HRR and
     digestion per quartet) over that time; on the three-atom system
     max|dJ|, max|dK| against the oracle's ordered sweep, whose time (J and
@@ -265,47 +274,53 @@ def split_jk_block(cpu: bool = True, cluster: bool = True) -> dict:
             t = time.perf_counter()
             plan = hjk.hjk_launches(s.basis, s.D, tau=1e-12, screen=screen)
             t_plan = time.perf_counter() - t
-            b = hjk.HJKBuild(s.basis, s.D, screen=screen, plan=plan)
-            b.run(hjk.STREAMS)
-            torch.cuda.synchronize()
-            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            reps = 3
-            e0.record()
-            for _ in range(reps):
+            for form, given in (("plan", plan), ("default", None)):
+                b = hjk.HJKBuild(s.basis, s.D, screen=screen, plan=given)
                 b.run(hjk.STREAMS)
-            e1.record()
-            torch.cuda.synchronize()
-            ms_eager = e0.elapsed_time(e1) / reps
-            b.capture(hjk.STREAMS)
-            b.replay()
-            torch.cuda.synchronize()
-            e0.record()
-            for _ in range(reps):
+                torch.cuda.synchronize()
+                e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                reps = 3
+                e0.record()
+                for _ in range(reps):
+                    b.run(hjk.STREAMS)
+                e1.record()
+                torch.cuda.synchronize()
+                ms_eager = e0.elapsed_time(e1) / reps
+                b.capture(hjk.STREAMS)
                 b.replay()
-            e1.record()
-            torch.cuda.synchronize()
-            ms_graph = e0.elapsed_time(e1) / reps
-            # the faster of the two forms is the build's time (the graph's
-            # four branches run slower than eager streams on the larger system)
-            ms = min(ms_graph, ms_eager)
-            X[screen] = b.X.cpu().numpy()
-            fl = b.flops
-            r[screen] = {"ms_per_build": ms, "timed_as": "graph" if ms_graph <= ms_eager else "eager",
-                         "ms_per_build_graph": ms_graph, "ms_per_build_eager": ms_eager,
-                         "launches": len(plan.launches), "quartets_visited":
-                         plan.counts()["quartets"], "quartets_computed": b.quartets_computed,
-                         "plan_s": t_plan,
-                         "roofline": {"bound": "fp64_valu", "achieved": fl / ms / 1e9,
-                                      "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                                      "frac": fl / ms / 1e9 / FP64_PEAK_TFLOPS, "gflop": fl / 1e9}}
+                torch.cuda.synchronize()
+                e0.record()
+                for _ in range(reps):
+                    b.replay()
+                e1.record()
+                torch.cuda.synchronize()
+                ms_graph = e0.elapsed_time(e1) / reps
+                # the faster of the two is the build's time (the planned form's graph of
+                # thousands of launches runs slower than eager streams on the larger system)
+                ms = min(ms_graph, ms_eager)
+                X[screen, form] = b.X.cpu().numpy()
+                fl = b.flops
+                q = {"ms_per_build": ms, "timed_as": "graph" if ms_graph <= ms_eager else "eager",
+                     "ms_per_build_graph": ms_graph, "ms_per_build_eager": ms_eager,
+                     "launches": len(plan.launches) if given else len(b.builder.launches),
+                     "quartets_computed": b.quartets_computed,
+                     "roofline": {"bound": "fp64_valu", "achieved": fl / ms / 1e9,
+                                  "kernel": "fj_hs_<rep>_k" if given else "fj_c_<cls>_k",
+                                  "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+                                  "frac": fl / ms / 1e9 / FP64_PEAK_TFLOPS, "gflop": fl / 1e9}}
+                if given:
+                    r[screen] = {**q, "quartets_visited": plan.counts()["quartets"], "plan_s": t_plan}
+                else:
+                    r[screen]["default"] = q
         if key == "c1_3atom":
             sys.path.insert(0, str(ROOT / "tests"))
             from oracle import oracle as O
             t = time.perf_counter()
             Jo, Ko = O.fock_ordered(s.basis, s.D)
             t = time.perf_counter() - t
-            r["max_dJ_vs_oracle"] = float(np.abs(X["j"] - Jo).max())
-            r["max_dK_vs_oracle"] = float(np.abs(X["k"] - Ko).max())
+            for form, name in (("plan", ""), ("default", "_default")):
+                r[f"max_dJ_vs_oracle{name}"] = float(np.abs(X["j", form] - Jo).max())
+                r[f"max_dK_vs_oracle{name}"] = float(np.abs(X["k", form] - Ko).max())
             if cpu:
                 r["cpu_baseline"] = {"value": 1.0 / t, "unit": "J+K builds/s", "cores": O.threads(),
                                      "kind": "port",
@@ -398,7 +413,7 @@ def df_block(cpu: bool = True) -> dict:
                              "n_aux": aux.n_aux, "metric_ms": ms_m, "eri3_ms": ms_3,
                              "eri3_integrals_per_s": s.basis.n_ao * (s.basis.n_ao + 1) / 2 * aux.n_aux
                              / ms_3 * 1e3,
-                             "roofline": {"bound": "fp64_valu", "kernel": "fj_dfloop_k (eri3)",
+                             "roofline": {"bound": "fp64", "kernel": "fj_dfquad_k (eri3)",
                                           "achieved": fl3 / ms_3 / 1e9, "peak": FP64_PEAK_TFLOPS,
                                           "unit": "TFLOP/s", "frac": fl3 / ms_3 / 1e9 / FP64_PEAK_TFLOPS,
                                           "gflop": fl3 / 1e9, "metric_tflops": flm / ms_m / 1e9}}
@@ -521,8 +536,8 @@ def jk_block(steps, warmup):
 
 def c4_block(a) -> None:
     """The batched workload: the 64 C4 molecules (8-80 atoms, seeds 4 + i)
-    with their s,s,p,d shells (the f shells run on the loop-form kernel, far
-    too slow for this batch) in one builder: one launch per class pair (and
+    with their s,s,p,d shells (with the f shells, 45,402 AOs, the batch is
+    not timed) in one builder: one launch per class pair (and
     tier) for all of them, dealt to streams, captured in a graph. Timed:
     the FP64 batch, the production batch (mixed precision, the learned
     selector choosing tiers per build on the device, the FP32 tier where it
@@ -640,10 +655,8 @@ def cof_block(a) -> None:
 def c4f_block(a) -> None:
     """C4 molecules with their f shells, each built alone (FP64, the
     launches dealt to --streams streams, eager): one warm-up and `--steps` timed builds per molecule, beside the
-    same molecule built through d. The whole 64-molecule batch with f is not
-    timed: the f classes run on the loop-form kernels, which make the
-    11-atom molecule 17 times slower than through d, and the batch holds
-    molecules of up to 80 atoms (45,402 AOs in all)."""
+    same molecule built through d. The whole 64-molecule batch with f
+    (molecules of up to 80 atoms, 45,402 AOs in all) is not timed."""
     import torch
     from felizjueves_amd import native
     from felizjueves_amd.fock import FockBuilder
@@ -683,7 +696,7 @@ def c4f_block(a) -> None:
 def c4f_batch_block(a) -> None:
     """Chosen C4 molecules with their f shells in one batch builder (one
     launch per class pair for all of them, --streams streams, eager; the f classes
-    on the loop-form kernel): batched builds/s, and the first molecule
+    on the matrix-core kernel): batched builds/s, and the first molecule
     against its own single build."""
     import torch
     from felizjueves_amd import native
@@ -735,8 +748,8 @@ def main() -> None:
                                            "split-df"),
                     default="c2",
                     help="c4d: the 64-molecule batch (8-80 atoms, seeds 4+i) with s,s,p,d shells "
-                         "(with its f shells, 45,402 AOs, one build would take minutes on the "
-                         "matrix-core f kernels); cof: CO/cc-pVTZ through f (the matrix-core kernels); c4f: "
+                         "(with its f shells, 45,402 AOs, it is not timed); "
+                         "cof: CO/cc-pVTZ through f (the matrix-core kernels); c4f: "
                          "single C4 molecules with and without their f shells; c4f-batch: "
                          "chosen C4 molecules with f in one batch builder; gradient: the fused "
                          "two-electron gradient block alone; split-df: the split J / K and "
@@ -768,7 +781,7 @@ def main() -> None:
         torch.cuda.synchronize()
         lt = launch_times(plain, Dd, reps=1)
         Lp = plain.launches[int(np.argmax(lt[0]))]
-        print(json.dumps({"copy_bytes_each_way": n * 8, "dominant": f"fj_f_{''.join(map(str, Lp.cls))}_k",
+        print(json.dumps({"copy_bytes_each_way": n * 8, "dominant": kernel_name(Lp), "launch_ms": float(lt.max()),
                           "dominant_gflop": Lp.flops / 1e9}), flush=True)
         return
 
@@ -830,8 +843,8 @@ def main() -> None:
     roofline = {
         "bound": "fp64_valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
         "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None,
-        "kernel": f"fj_f_{''.join(map(str, Lp.cls))}_k<double>",
-        "note": ("compute-bound on FP64 VALU (no MFMA in this kernel); 78.6 TFLOP/s is MI355X's FP64 "
+        "kernel": kernel_name(Lp),
+        "note": ("FP64 VALU work (no MFMA in this kernel); 78.6 TFLOP/s is MI355X's FP64 "
                  "vector peak (equal to its FP64 matrix peak); achieved = algorithmic FLOPs of the "
                  "launch (hgp.Cost: VRR + boundary per primitive quartet, HRR + digestion per "
                  "quartet, no FMA credit) / mean duration of its eager launches (default plan, one "
@@ -844,7 +857,7 @@ def main() -> None:
         if t.get("kernel") == roofline["kernel"]:
             roofline["traffic"] = t["traffic_bytes"]
             roofline["traffic_note"] = (t["source"] + f", scaled by a 512 MiB copy (fetch x{t['fetch_scale']:.3f}, "
-                                        f"write x{t['write_scale']:.3f}); mostly the launch workspace")
+                                        f"write x{t['write_scale']:.3f}); {t['what']}")
     va = TUNED / f"valu_c2_{a.atoms}atom.json"
     if va.exists():
         t = json.loads(va.read_text())

@@ -7,7 +7,7 @@ kernels (`fj_metric_loop` / `fj_eri3_loop` and their per-class entries).
     AuxBasis.from_arrays(...)              an auxiliary basis (shells through i)
     metric_classes(aux) / metric_matrix(aux)          -> (P|Q) [n_aux, n_aux]
     eri3_classes(basis, aux) / eri3(basis, aux)       -> (mn|P) [n_ao, n_ao, n_aux]
-    flops_metric(aux) / flops_eri3(basis, aux)        -> the loop form's arithmetic
+    flops_metric(aux) / flops_eri3(basis, aux)        -> the kernels' arithmetic
     DfIntegrals(aux, basis).metric() / .eri3()         the tables staged once
 
 An aux primitive is a Hermite "pair" of one Gaussian: record (A, alpha, s =
@@ -171,27 +171,41 @@ def _cell_flops(la: int, lb: int, lc: int) -> int:
     return f
 
 
+QUAD_LMAX_AUX = 4   # aux shells of the matrix-core kernel (fj_dfquad.h); h and i run the loop form
+
+
+def _quad_flops(la: int, lb: int, lc: int) -> tuple[int, int]:
+    """The matrix-core kernel's arithmetic per record pair -- the tower (3 per
+    entry per level) and, for each bra Hermite index and aux component, 2 per
+    term of its E (parity box) -- and per bra record of a cell: 2 per E
+    product and 2 nab np nc."""
+    from .basis import cartesians
+    L = la + lb + lc
+    herm = lambda n: (n + 1) * (n + 2) * (n + 3) // 6   # |t| <= n   # noqa: E731
+    terms = sum((c[0] // 2 + 1) * (c[1] // 2 + 1) * (c[2] // 2 + 1) for c in cartesians(lc))
+    nab, nc, n_p = len(cartesians(la)) * len(cartesians(lb)), len(cartesians(lc)), herm(la + lb)
+    return sum(3 * herm(m) for m in range(1, L + 1)) + 2 * n_p * terms, 2 * nab * n_p * (nc + 1)
+
+
+def _class_flops(cls3, dc: DfClass, bra: str) -> int:
+    a = dc.arrays
+    k = "q" if bra == "p" else "p"
+    n_bra = (a[f"{bra}_rec1"] - a[f"{bra}_rec0"]).astype(np.int64)
+    n_rp = int((n_bra * (a[f"{k}_rec1"] - a[f"{k}_rec0"])).sum())
+    if cls3[2] > QUAD_LMAX_AUX:
+        return n_rp * _cell_flops(*cls3)
+    pair, rec = _quad_flops(*cls3)
+    return n_rp * pair + int(n_bra.sum()) * rec
+
+
 def flops_metric(aux: AuxBasis) -> int:
-    """The arithmetic of one metric_matrix call (_cell_flops over every
-    record pair of every aux shell pair)."""
-    tot = 0
-    for (lp, lq), dc in metric_classes(aux).items():
-        a = dc.arrays
-        n_rp = (a["p_rec1"] - a["p_rec0"]).astype(np.int64) * (a["q_rec1"] - a["q_rec0"])
-        tot += int(n_rp.sum()) * _cell_flops(lp, 0, lq)
-    return tot
+    """The arithmetic of one metric_matrix call, tiles' padding left out."""
+    return sum(_class_flops((lp, 0, lq), dc, "p") for (lp, lq), dc in metric_classes(aux).items())
 
 
 def flops_eri3(basis: Basis, aux: AuxBasis) -> int:
-    """The arithmetic of one eri3 call (_cell_flops over every record pair
-    of every cell)."""
-    classes, _ = eri3_classes(basis, aux)
-    tot = 0
-    for (la, lb, lp), dc in classes.items():
-        a = dc.arrays
-        n_rp = (a["ab_rec1"] - a["ab_rec0"]).astype(np.int64) * (a["p_rec1"] - a["p_rec0"])
-        tot += int(n_rp.sum()) * _cell_flops(la, lb, lp)
-    return tot
+    """The arithmetic of one eri3 call, tiles' padding left out."""
+    return sum(_class_flops(c, dc, "ab") for c, dc in eri3_classes(basis, aux)[0].items())
 
 
 def _p(t):

@@ -175,16 +175,26 @@ def flops_per_prim_quartet(cls) -> int:
 
 
 def flops(stream: GfStream) -> int:
-    """The stream's arithmetic (flops_per_prim_quartet over every primitive
-    quartet of every launch)."""
+    """The stream's arithmetic in the matrix-core kernel's formulation
+    (fj_gfquad.h), its tiles' padding and recomputed tables left out: per
+    primitive quartet the tower (3 per entry per level), the two products
+    with it and 18 per bra element (ab, t); per quartet the bra primitives'
+    weights (2 nab ncd nt and the E products) and the ket primitives', and 17
+    per ket element (cd, u)."""
     tot = 0
-    cache: dict = {}
     for L in stream.launches:
+        la, lb, lc, ld = L.cls
         b, k = stream.sides[L.bra], stream.sides[L.ket]
         nq = b.n * (b.n + 1) // 2 if L.diag else b.n * k.n
-        if L.cls not in cache:
-            cache[L.cls] = flops_per_prim_quartet(L.cls)
-        tot += nq * b.degree * k.degree * cache[L.cls]
+        cart = lambda x: (x + 1) * (x + 2) // 2   # noqa: E731
+        herm = lambda x: (x + 1) * (x + 2) * (x + 3) // 6   # |t| <= x   # noqa: E731
+        nab, ncd, Lt = cart(la) * cart(lb), cart(lc) * cart(ld), sum(L.cls) + 1
+        nt, nt1, nu, nu1 = herm(la + lb), herm(la + lb + 1), herm(lc + ld), herm(lc + ld + 1)
+        tower = sum(3 * herm(m) for m in range(1, Lt + 1))
+        pq = 2 * nab * nu * nt1 + 2 * ncd * nt * nu1 + 18 * nab * nt1 + tower
+        bra = 2 * nab * nt * (ncd + 1)
+        ket = 2 * ncd * nu * (nab + 1) + 17 * ncd * nu1
+        tot += nq * (b.degree * k.degree * pq + b.degree * bra + k.degree * ket)
     return tot
 
 
