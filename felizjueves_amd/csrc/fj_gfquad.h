@@ -6,7 +6,7 @@
 // quartets). With i over the bra's primitive pairs and j over the ket's,
 //
 //   Wk_j[ab][u] = (-1)^|u| sum_cd w E^{cd}_u(j)       once per j and wavefront
-//   Wb_i[cd][t] = sum_ab w E^{ab}_t(i)                once per i and workgroup
+//   Wb_i[cd][t] = sum_ab w E^{ab}_t(i)                once per i and pass over j
 //   Y_ij[ab][t] = sum_u Wk_j[ab][u] [t + u]_ij        gA, gB += sum dE^{ab}_t(i) Y_ij
 //   X_j[cd][u] += sum_i sum_t Wb_i[cd][t] [t + u]_ij  gC, gD once per j
 //
@@ -16,7 +16,8 @@
 // primitives and X is summed over i in the accumulators, where the loop form
 // forms all of it per primitive quartet: at (dd|dd) about 300 thousand
 // operations per primitive quartet are left, nearly all in the two products
-// with [t + u].
+// with [t + u]. A pass is four j (one per wavefront), and a batch's tables and
+// Wb are formed for all IB rows, also where the item has fewer.
 //
 // Wavefronts take different j (or, for one or two j, different i); the i are
 // taken IB at a time: their E tables and Wb by the workgroup, then each
@@ -31,10 +32,10 @@
 // Measured on MI355X, every class of the s,s,p,d 8-atom gradient alone (29.8
 // million primitive quartets): 666 ms in the loop form, 55 ms here, and 22.3
 // -> 6.4 ms for the three-atom one; e.g. (dd|dd) 32.2 -> 4.8 ms, (sp|dd) 75.8
-// -> 2.8 ms, (ss|sp) 4.8 -> 1.1 ms. The matrix cores are busy 27 to 32% of the
-// time of the classes with a d pair on the ket; about as many cycles go to
-// the towers' and the last stage's index and FP64 instructions (12 per matrix
-// step at (dd|dd)), the rest to waits for LDS.
+// -> 2.8 ms, (ss|sp) 4.8 -> 1.1 ms. The matrix cores are busy 13 to 26% of the
+// time of the classes with a d shell in the ket; to each matrix step come 8 to
+// 39 VALU instructions of the towers and the last stage (12.5 at (dd|dd)), and
+// the wavefronts wait in 15 to 28% of their cycles.
 //
 // The includer provides fj_device.h (the device one, or the CPU emulation)
 // and fj_gfloop.h.

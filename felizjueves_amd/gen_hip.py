@@ -1611,7 +1611,7 @@ def emit_quartet_staged(cls, split: bool = False) -> str:
 # quartets, boundaries summed in LDS, HRR and digestion once per quartet.
 
 COOP_LDS = 159 * 1024   # of a CU's 160 KB
-COOP_NQ_MAX = 32
+COOP_NQ_MAX = 8         # quartets of a wavefront, at most
 
 
 def coop_tune(cls) -> tuple[int, int, int, int]:
@@ -1666,7 +1666,7 @@ def coop_shape(cls) -> dict:
     wt = max(chunk * 65, qw * (sa * nb * xs + no))
     fixed = 8 * (MAX_PRIM_PAIRS * 9 + 4 * wt + na * nb)
     nq = (COOP_LDS // wgs - fixed) // (4 * (8 * reg + 32))
-    nq = int(max(1, min(COOP_NQ_MAX // 4, nq)))
+    nq = int(max(1, min(COOP_NQ_MAX, nq)))
     qw = min(qw, nq)
     return dict(na=na, nb=nb, nc=nc, nd=nd, ne=ne, nf=nf, reg=reg, xs=xs, no=no, qw=qw, sa=sa, wt=wt,
                 nq=nq, live=live, wgs=wgs, chunk=chunk)
