@@ -1,6 +1,7 @@
 // fj_gfloop.hip -- the launcher of the fused two-electron gradient kernel
 // (fj_gfloop.h) with the upstream gf_ parameter list; the per-class entries
 // fj_gf_<la><lb><lc><ld> (gen/gf_entries.hip) call it.
+#include <algorithm>
 #include "fj_device.h"
 #include "fj_gfloop.h"
 #include "gen/gq_table.h"
@@ -19,6 +20,16 @@ static int fj_gf_chunk(long long n_q, int n_pq, int B) {
     int chunk = (int)((n_pq + pieces - 1) / pieces);
     chunk = (chunk + B - 1) / B * B;
     return chunk < n_pq ? chunk : n_pq;
+}
+
+// The same for the matrix-core kernel (gradient.quad_chunk), `rows` bra
+// primitives to a wavefront's step.
+static int fj_gq_chunk(long long n_q, int k_ab, int k_cd, int rows) {
+    const long long n_pq = (long long)k_ab * k_cd, pieces = n_q >= GF_ITEMS ? 1 : (GF_ITEMS + n_q - 1) / n_q;
+    rows *= k_cd == 1 ? 8 : k_cd == 2 ? 4 : 2;
+    const long long pj = std::min<long long>(pieces, (k_cd + 3) / 4);
+    const long long pi = std::min<long long>((pieces + pj - 1) / pj, (k_ab + rows - 1) / rows);
+    return (int)((n_pq + pi * pj - 1) / (pi * pj));
 }
 
 // The kernel of a launch at `threads` lanes: at 256 (the default width) the
@@ -54,9 +65,7 @@ extern "C" int fj_gf_loop(hipStream_t s, int la, int lb, int lc, int ld, int thr
     const long long n_q = diag ? (long long)n_bra * (n_bra + 1) / 2 : (long long)n_bra * n_ket;
     const int n_pq = k_ab * k_cd;
     if (fj_gfquad_t quad = fj_gf_quad(la, lb, lc, ld, threads)) {
-        // few quartets: their rows of primitives (one bra primitive each) in pieces
-        const int pieces = (int)(n_q >= GF_ITEMS ? 1 : (GF_ITEMS + n_q - 1) / n_q);
-        const int chunk = (k_ab + pieces - 1) / pieces * k_cd;
+        const int chunk = fj_gq_chunk(n_q, k_ab, k_cd, fj_gfquad_rows(la, lb, lc, ld));
         const FjGfArgs g{la, lb, lc, ld, n_bra, n_ket, k_ab, k_cd, n_atom, n_ao, diag, chunk, bra_prim, AB, bra_sh,
                          bra_ao, bra_at, ket_prim, CD, ket_sh, ket_ao, ket_at, D, G};
         const long long n_items = n_q * ((n_pq + chunk - 1) / chunk);

@@ -16,8 +16,8 @@
 // primitives and X is summed over i in the accumulators, where the loop form
 // forms all of it per primitive quartet: at (dd|dd) about 300 thousand
 // operations per primitive quartet are left, nearly all in the two products
-// with [t + u]. A pass is four j (one per wavefront), and a batch's tables and
-// Wb are formed for all IB rows, also where the item has fewer.
+// with [t + u]. A pass is four j (one per wavefront). A quartet cut into
+// pieces (few quartets) is cut into ranges of j first, then of i.
 //
 // Wavefronts take different j (or, for one or two j, different i); the i are
 // taken IB at a time: their E tables and Wb by the workgroup, then each
@@ -72,7 +72,7 @@ struct Gq {
     // X += Wb [t + u] (rows cd, columns u, over (i, t)), of Wb and of Wk
     static constexpr int MY = gq_up(NAB, 16), NY = gq_up(IBW * NT1, 16), KY = gq_up(NU, 4);
     static constexpr int MX = gq_up(NCD, 16), NX = gq_up(NU1, 16), KX = gq_up(IBW * NT, 4);
-    static constexpr int NWB = gq_up(IB * NT, 16), KWB = gq_up(NAB, 4);
+    static constexpr int KWB = gq_up(NAB, 4);
     static constexpr int NWK = gq_up(NU, 16), KWK = gq_up(NCD, 4);
     // one axis's table (value and its derivatives by the two centres), [i][j][t]
     static constexpr int TB = (LA + 1) * (LB + 1) * (LAB + 2), TK = (LC + 1) * (LD + 1) * (LCD + 2);
@@ -247,7 +247,12 @@ __global__ void __launch_bounds__(GQ_THREADS, (LA + LB + LC + LD == 8 ? 1 : 2)) 
         FjGfArgs g = g0;
         int pq0, pq1, bra, ket;
         const double deg = fj_gf_item(g, jobs, n_jobs, q0, pq0, pq1, bra, ket);
-        const int k_cd = g.k_cd, i_lo = pq0 / k_cd, i_hi = (pq1 - 1) / k_cd;   // rows with work
+        // piece c of the quartet's n: a range of columns j and one of rows i
+        const int k_cd = g.k_cd, n = (g.k_ab * k_cd + g.chunk - 1) / g.chunk, c = pq0 / g.chunk;
+        const int n4 = (k_cd + 3) / 4, pj = min(n, n4), pi = min(n / pj, g.k_ab), cj = c % pj, ci = c / pj;
+        if (ci >= pi) continue;   // uniform; the pieces before have it all
+        const int j0 = 4 * (int)((long long)cj * n4 / pj), j1 = min(k_cd, 4 * (int)((long long)(cj + 1) * n4 / pj));
+        const int i_lo = (int)((long long)ci * g.k_ab / pi), i_hi = (int)((long long)(ci + 1) * g.k_ab / pi) - 1;
         __syncthreads();   // the previous item's readers of w are done
         {
             const size_t n = (size_t)g.n_ao;
@@ -268,13 +273,13 @@ __global__ void __launch_bounds__(GQ_THREADS, (LA + LB + LC + LD == 8 ? 1 : 2)) 
         double gA[3] = {0.0, 0.0, 0.0}, gB[3] = {0.0, 0.0, 0.0};
         double gC[3] = {0.0, 0.0, 0.0}, gD[3] = {0.0, 0.0, 0.0};
         // wavefronts over j, and over i where there are fewer than three j
-        const int WJ = k_cd >= 3 ? 4 : k_cd, WI = GQ_WAVES / WJ, wj = wave % WJ, wi = wave / WJ;
+        const int WJ = min(4, j1 - j0 == 3 ? 4 : j1 - j0), WI = GQ_WAVES / WJ, wj = wave % WJ, wi = wave / WJ;
         __syncthreads();
 
-        for (int jb = 0; jb < k_cd; jb += WJ) {
+        for (int jb = j0; jb < j1; jb += WJ) {
             const int j = jb + wj;
-            const bool jv = j < k_cd;
-            const double* __restrict__ rk = kp + (jv ? j : 0) * GF_REC;
+            const bool jv = j < j1;
+            const double* __restrict__ rk = kp + (jv ? j : j0) * GF_REC;
             const double qz = rk[6], Qx = rk[0], Qy = rk[1], Qz = rk[2];
             // the ket's axis tables (U in the x axis), then Wk as A operands
             if (lane < 3 * (LC + 2)) {
@@ -327,23 +332,24 @@ __global__ void __launch_bounds__(GQ_THREADS, (LA + LB + LC + LD == 8 ? 1 : 2)) 
                 for (int n = 0; n < NX; ++n) xa[m][n] = fj_v4d{0.0, 0.0, 0.0, 0.0};
 
             for (int ib = i_lo; ib <= i_hi; ib += IB) {
+                const int nr = min(IB, i_hi - ib + 1);   // the batch's rows
                 __syncthreads();   // the previous batch's readers of eb and wb are done
-                for (int r = tid; r < IB * 3 * (LA + 2); r += GQ_THREADS) {
+                for (int r = tid; r < nr * 3 * (LA + 2); r += GQ_THREADS) {
                     const int bk = r / (LA + 2), b = bk / 3, k = bk - 3 * b;
-                    const double* __restrict__ rb = bp + min(ib + b, i_hi) * GF_REC;
+                    const double* __restrict__ rb = bp + (ib + b) * GF_REC;
                     gq_rows<LA, LB>(S.wb + bk * Q::EB, r - bk * (LA + 2), rb[6], rb[3 + k], rb[3 + k] + AB[k],
                                        k == 0 ? rb[7] : 1.0);
                 }
                 __syncthreads();
-                for (int r = tid; r < IB * 3 * TB; r += GQ_THREADS) {
-                    const int bk = r / TB, i = min(ib + bk / 3, i_hi);
+                for (int r = tid; r < nr * 3 * TB; r += GQ_THREADS) {
+                    const int bk = r / TB, i = ib + bk / 3;
                     gq_entry<LA, LB>(S.eb + bk * TB * 3, S.wb + bk * Q::EB, r - bk * TB, 2.0 * bp[i * GF_REC + 8],
                                      2.0 * bp[i * GF_REC + 9]);
                 }
                 __syncthreads();
                 // Wb of the batch: rows cd, columns (i, t), over ab
-                for (int n = wave; n < Q::NWB; n += GQ_WAVES) {
-                    const int col = min(16 * n + l16, IB * NT - 1), b = col / NT, t = col - b * NT;
+                for (int n = wave; 16 * n < nr * NT; n += GQ_WAVES) {
+                    const int col = min(16 * n + l16, nr * NT - 1), b = col / NT, t = col - b * NT;
                     const double* __restrict__ e = S.eb + b * 3 * TB * 3;
                     fj_v4d acc[MX];
 #pragma unroll
@@ -362,17 +368,18 @@ __global__ void __launch_bounds__(GQ_THREADS, (LA + LB + LC + LD == 8 ? 1 : 2)) 
 #pragma unroll
                         for (int v = 0; v < 4; ++v) {
                             const int cd = 16 * m + l4 + 4 * v;
-                            if (16 * n + l16 < IB * NT && cd < NCD) S.wb[col * WBS + cd] = acc[m][v];
+                            if (16 * n + l16 < nr * NT && cd < NCD) S.wb[col * WBS + cd] = acc[m][v];
                         }
                 }
                 __syncthreads();
                 for (int s = wi; s < Q::SB; s += WI) {
                     const int i0 = ib + s * IBW;
                     if (!jv || i0 > i_hi) break;   // uniform over the wavefront
-                    // seeds (zero outside the item's primitive quartets), then the towers' levels
+                    const int last = min(IBW - 1, i_hi - i0);   // the step's last row with tables
+                    // seeds (zero past the last row), then the towers' levels
                     if (lane < IBW) {
-                        const int i = min(i0 + lane, i_hi), pq = i * k_cd + j;
-                        const bool in = i0 + lane <= i_hi && pq >= pq0 && pq < pq1;
+                        const int i = i0 + min(lane, last);
+                        const bool in = lane <= last;
                         const double* __restrict__ rb = bp + i * GF_REC;
                         const double p = rb[6], x = rb[0] - Qx, y = rb[1] - Qy, z = rb[2] - Qz;
                         const double rho = p * qz / (p + qz);
@@ -420,7 +427,7 @@ __global__ void __launch_bounds__(GQ_THREADS, (LA + LB + LC + LD == 8 ? 1 : 2)) 
                             double av[MX];
 #pragma unroll
                             for (int m = 0; m < MX; ++m) {
-                                const double t = wb[min(k, IBW * NT - 1) * WBS + min(16 * m + l16, NCD - 1)];
+                                const double t = wb[min(k, (last + 1) * NT - 1) * WBS + min(16 * m + l16, NCD - 1)];
                                 av[m] = k < IBW * NT ? t : 0.0;
                             }
 #pragma unroll
@@ -437,6 +444,7 @@ __global__ void __launch_bounds__(GQ_THREADS, (LA + LB + LC + LD == 8 ? 1 : 2)) 
                     // up and spilling)
 #pragma unroll
                     for (int n = 0; n < NY; ++n) {
+                        if (16 * n >= (last + 1) * NT1) break;   // uniform
                         __asm__ volatile("" ::: "memory");
                         fj_v4d y[MY];
 #pragma unroll
@@ -449,7 +457,7 @@ __global__ void __launch_bounds__(GQ_THREADS, (LA + LB + LC + LD == 8 ? 1 : 2)) 
                             for (int m = 0; m < MY; ++m) y[m] = fj_mfma_f64_16x16x4(wk[m][ks], bv, y[m]);
                         }
                         const int col = 16 * n + l16, b = min(col, IBW * NT1 - 1) / NT1, t = min(col, IBW * NT1 - 1) % NT1;
-                        const double* __restrict__ e = S.eb + (s * IBW + b) * 3 * TB * 3;
+                        const double* __restrict__ e = S.eb + (s * IBW + min(b, last)) * 3 * TB * 3;
 #pragma unroll
                         for (int m = 0; m < MY; ++m) {
                             __asm__ volatile("" ::: "memory");

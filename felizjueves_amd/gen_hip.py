@@ -940,7 +940,8 @@ def emit_gf_entries() -> str:
 
 def generate_gfquad(out: Path = GEN) -> list[Path]:
     """gq_<cls>.hip, the matrix-core gradient kernel's launch of one class
-    each, and gq_table.h, their dispatch."""
+    each, and gq_table.h, their dispatch and the rows of a wavefront's step."""
+    from .gradient import quad_rows
     out.mkdir(parents=True, exist_ok=True)
     sig = "(hipStream_t s, unsigned grid, const FjGfArgs& g, const FjGfJob* jobs, int n_jobs, long long n_items)"
     files, texts = [], {}
@@ -949,6 +950,7 @@ def generate_gfquad(out: Path = GEN) -> list[Path]:
         texts[f"gq_{n}.hip"] = (
             "// generated by felizjueves_amd/gen_hip.py -- matrix-core gradient kernel\n"
             '#include "../fj_device.h"\n#include "../fj_gfloop.h"\n#include "../fj_gfquad.h"\n\n'
+            f"static_assert(Gq<{', '.join(map(str, c))}>::IBW == {quad_rows(c)}, \"rows of a step\");\n\n"
             f"int fj_gfquad_{n}{sig.replace('const FjGfArgs& g', 'const void* g')} {{\n"
             f"    hipLaunchKernelGGL((fj_gfquad_k<{', '.join(map(str, c))}>), dim3(grid), dim3(GQ_THREADS), 0, s,\n"
             "                       *static_cast<const FjGfArgs*>(g), jobs, n_jobs, n_items);\n"
@@ -961,7 +963,11 @@ def generate_gfquad(out: Path = GEN) -> list[Path]:
     L += ["", "static inline fj_gfquad_t fj_gfquad_for(int la, int lb, int lc, int ld) {",
           "    switch (((la * 4 + lb) * 4 + lc) * 4 + ld) {"]
     L += [f"        case {((c[0] * 4 + c[1]) * 4 + c[2]) * 4 + c[3]}: return fj_gfquad_{cls_name(c)};" for c in gf_classes()]
-    L += ["        default: return nullptr;   // a class outside the stream", "    }", "}", ""]
+    L += ["        default: return nullptr;   // a class outside the stream", "    }", "}", "",
+          "static inline int fj_gfquad_rows(int la, int lb, int lc, int ld) {",
+          "    switch (((la * 4 + lb) * 4 + lc) * 4 + ld) {"]
+    L += [f"        case {((c[0] * 4 + c[1]) * 4 + c[2]) * 4 + c[3]}: return {quad_rows(c)};" for c in gf_classes()]
+    L += ["        default: return 1;", "    }", "}", ""]
     texts["gq_table.h"] = "\n".join(L)
     for fname, text in texts.items():
         p = out / fname

@@ -215,6 +215,31 @@ JOB_DTYPE = np.dtype([("bra_row", "<i4"), ("ket_row", "<i4"), ("n_bra", "<i4"), 
                       ("bra_prim", "<i8"), ("ket_prim", "<i8"), ("q0", "<i8")])   # FjGfJob
 
 
+@lru_cache(maxsize=None)
+def quad_rows(cls) -> int:
+    """Bra primitives of a wavefront's step in the matrix-core kernel
+    (fj_gfquad.h IBW, checked against it where the kernels are built)."""
+    herm = lambda n: (n + 1) * (n + 2) * (n + 3) // 6   # noqa: E731
+    nr, nt1 = herm(sum(cls) + 1), herm(cls[0] + cls[1] + 1)
+    return {4: 16 if nr <= 20 else 8 if nr <= 56 else 4, 10: 6 if nr <= 56 else 3, 20: 3}.get(nt1, 1)
+
+
+def quad_chunk(cls, k_ab: int, k_cd: int, pieces: int) -> int:
+    """The chunk that splits a quartet into about `pieces` for the matrix-core
+    kernel, which takes a piece as a range of the ket's primitives, four to a
+    pass, and one of the bra's rows (fj_gfquad.h, whose pieces follow from the
+    chunk): the ket's ranges first, and of the rows no fewer than two steps of
+    the workgroup's wavefronts. The rows of a step run side by side, so fewer
+    of them make more pieces, each with its tables and twelve atomics, and no
+    shorter one: H2O/STO-3G 0.24 -> 0.11 ms, one atom s,s,p,d 1.08 -> 0.65, two
+    2.51 -> 1.33, three 3.79 -> 2.88 (pieces down to single rows: 2.48 ms for
+    the one atom where rows alone were cut, 1.68 in the loop form)."""
+    pj = min(pieces, -(-k_cd // 4))
+    rows = quad_rows(cls) * (2 if k_cd > 2 else 4 if k_cd == 2 else 8)   # (wavefronts beyond the ket's primitives take rows)
+    pi = min(-(-pieces // pj), -(-k_ab // rows))
+    return -(-k_ab * k_cd // (pi * pj))
+
+
 class GpuGfRunner:
     """The stream's sides on the device, reused across densities; `run`
     launches every class into a zeroed G on `stream`.
@@ -245,8 +270,9 @@ class GpuGfRunner:
                     self.fns[L.cls] = fn
             return
         # the sides concatenated: rows and record offsets per side
-        rows = np.concatenate([[0], np.cumsum([sd.n for sd in stream_.sides])]).astype(np.int64)
-        recs = np.concatenate([[0], np.cumsum([sd.prim.size for sd in stream_.sides])]).astype(np.int64)
+        sides = stream_.sides
+        rows = np.concatenate([[0], np.cumsum([sd.n for sd in sides])]).astype(np.int64).tolist()
+        recs = np.concatenate([[0], np.cumsum([sd.prim.size for sd in sides])]).astype(np.int64).tolist()
         cat = lambda k: np.concatenate([getattr(sd, k).reshape(sd.n, -1) for sd in stream_.sides])  # noqa: E731
         self.cat = {"prim": native.to_dev(np.concatenate([sd.prim.ravel() for sd in stream_.sides])),
                     **{k: native.to_dev(np.ascontiguousarray(cat(k))) for k in ("sep", "sh", "ao", "at")}}
@@ -256,29 +282,29 @@ class GpuGfRunner:
         self.classes = []
         lib.fj_gf_batch.restype = C.c_int
         for cls, Ls in sorted(by.items()):
-            jobs = np.zeros(len(Ls), dtype=JOB_DTYPE)
-            nq = [stream_.sides[L.bra].n * (stream_.sides[L.bra].n + 1) // 2 if L.diag
-                  else stream_.sides[L.bra].n * stream_.sides[L.ket].n for L in Ls]
-            max_pq = max(stream_.sides[L.bra].degree * stream_.sides[L.ket].degree for L in Ls)
+            jobs = []
+            dims = [(b.n, k.n, b.degree, k.degree) for b, k in ((sides[L.bra], sides[L.ket]) for L in Ls)]
+            nq = [nb * (nb + 1) // 2 if L.diag else nb * nk for L, (nb, nk, _, _) in zip(Ls, dims)]
+            max_pq = max(kab * kcd for _, _, kab, kcd in dims)
             th = self.threads.get(cls, default_threads(cls))
             B = int(lib.fj_gf_batch(*[C.c_int(x) for x in cls], C.c_int(max_pq), C.c_int(th)))
             # a class of few quartets splits each quartet's primitive quartets
-            # into pieces so that about ITEMS items fill the chip: whole rows
-            # (one bra primitive pair each) for the matrix-core kernel,
-            # multiples of the loop form's batch B otherwise
+            # into pieces so that about ITEMS items fill the chip: ranges of
+            # its ket and bra primitives for the matrix-core kernel
+            # (quad_chunk), multiples of the loop form's batch B otherwise
             pieces = max(1, -(-ITEMS // sum(nq)))
             q0 = 0
-            for j, L in enumerate(Ls):
-                b, k = stream_.sides[L.bra], stream_.sides[L.ket]
-                n_pq = b.degree * k.degree
-                if th == QUAD_THREADS:
-                    chunk = -(-b.degree // pieces) * k.degree
+            for j, (L, (nb, nk, kab, kcd)) in enumerate(zip(Ls, dims)):
+                n_pq = kab * kcd
+                if pieces == 1:
+                    chunk = n_pq
+                elif th == QUAD_THREADS:
+                    chunk = quad_chunk(cls, kab, kcd, pieces)
                 else:
-                    chunk = n_pq if pieces == 1 else min(n_pq, -(-(-(-n_pq // pieces)) // B) * B)
-                jobs[j] = (rows[L.bra], rows[L.ket], b.n, k.n, b.degree, k.degree, L.diag, chunk,
-                           recs[L.bra], recs[L.ket], q0)
+                    chunk = min(n_pq, -(-(-(-n_pq // pieces)) // B) * B)
+                jobs.append((rows[L.bra], rows[L.ket], nb, nk, kab, kcd, L.diag, chunk, recs[L.bra], recs[L.ket], q0))
                 q0 += nq[j] * -(-n_pq // chunk)
-            jd = native.to_dev(np.frombuffer(jobs.tobytes(), dtype=np.uint8))
+            jd = native.to_dev(np.frombuffer(np.array(jobs, dtype=JOB_DTYPE).tobytes(), dtype=np.uint8))
             self.classes.append((cls, jd, len(Ls), q0, max_pq))
         self.fj_gf_jobs = lib.fj_gf_jobs
         self.fj_gf_jobs.restype = C.c_int

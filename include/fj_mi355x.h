@@ -1996,7 +1996,8 @@ int fj_gf_batch(int la, int lb, int lc, int ld, int n_pq, int threads);
  * record offset bra_prim (doubles), and its ket likewise. A job's work items
  * are its quartets (in the order of one fj_gf_<cls> launch of those sides),
  * each split into ceil(k_ab k_cd / chunk) items of `chunk` primitive
- * quartets; job j owns items q0 .. q0 + (its count) - 1 of n_items. jobs
+ * quartets (of about as many at 256 lanes: a range of the bra's primitive
+ * pairs by one of the ket's); job j owns items q0 .. q0 + (its count) - 1 of n_items. jobs
  * (device memory) are sorted by q0, q0[0] = 0, chunk >= 1, and max_pq bounds
  * every job's k_ab k_cd. The table is trusted as the host stream builds it
  * (gradient.py); the per-class entries are the validated single launches.

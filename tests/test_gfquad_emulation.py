@@ -94,14 +94,32 @@ def deep_exe(tmp_path_factory):
                                                       (0, 2, 0, 2), (0, 2, 2, 2)])
 
 
-@pytest.mark.parametrize("name", list(DEEP))
-def test_matrix_core_gradient_of_deep_contractions(name, deep_exe, tmp_path):
+@pytest.mark.parametrize("name,pieces", [("s", 1), ("s", 9), ("p", 1), ("p", 20), ("d", 1), ("d", 5), ("sd", 1), ("sd", 3)])
+def test_matrix_core_gradient_of_deep_contractions(name, pieces, deep_exe, tmp_path):
     """Several batches of a bra's rows (the tables and weights in LDS
     rewritten) and several passes over the ket's primitives, the last of them
-    with idle wavefronts (5, 9, 25 and 81 primitives by fours, 3 alone)."""
+    with idle wavefronts (5, 9, 25 and 81 primitives by fours, 3 alone); whole
+    quartets, and pieces that cut the ket's primitives alone and the bra's
+    rows too, some of them left empty."""
     (l0, n0), (l1, n1) = DEEP[name]
     e = lambda n, x: tuple(x * 1.7 ** -np.arange(n))   # noqa: E731
     c = lambda n: tuple(0.6 - 0.05 * np.arange(n))   # noqa: E731
     basis = Basis([_shell(l0, (0.1, -0.2, 0.3), e(n0, 3.0), c(n0)), _shell(l1, (-0.7, 0.8, 0.4), e(n1, 0.9), c(n1))])
     D = closed_shell_density(np.random.default_rng(3), basis.n_ao, min(3, basis.n_ao - 1))
-    _gradient(deep_exe, tmp_path, basis, [0, 1], D, 1)
+    _gradient(deep_exe, tmp_path, basis, [0, 1], D, pieces)
+
+
+@pytest.mark.parametrize("cls", [(0, 0, 0, 0), (0, 1, 0, 2), (1, 1, 2, 2), (2, 2, 2, 2)])
+@pytest.mark.parametrize("k_ab,k_cd,pieces", [(36, 36, 37), (1, 36, 37), (36, 1, 37), (5, 9, 4), (7, 5, 12), (3, 9, 9), (4, 4, 1),
+                                              (81, 2, 2048)])
+def test_pieces_cut_the_ket_before_the_rows(cls, k_ab, k_cd, pieces):
+    """The pieces that a chunk makes in the kernel are ranges of whole passes
+    over the ket first, then of at least two steps' rows (but for a last
+    remainder's share)."""
+    n = -(-k_ab * k_cd // GR.quad_chunk(cls, k_ab, k_cd, pieces))   # as fj_gfquad.h has it
+    pj = min(n, -(-k_cd // 4))
+    pi = min(n // pj, k_ab)
+    rows = 2 * GR.quad_rows(cls) * (4 if k_cd == 1 else 2 if k_cd == 2 else 1)
+    assert pj == min(pieces, -(-k_cd // 4)) and pj * pi <= n
+    assert pj * pi <= pieces + pj - 1 and pi <= -(-k_ab // rows)
+    assert pj * pi >= min(pieces, pj * -(-k_ab // rows)) or pi == n // pj
