@@ -273,3 +273,38 @@ extern "C" void fj_plan_free(FjPlanResult* out) {
         out->kets[t] = nullptr;
     }
 }
+
+// Items for the cooperative kernels (host code): the items of the first bra
+// chunks, in their order, each with its first-chunk kets, cut into equal
+// pieces of at most `batch`.
+extern "C" int fj_coop_items(const int* work, int n_work, const int* ket_list, int n_list, int batch,
+                             int* out_work, int* out_parent, int* out_kets, long long* counts) {
+    if (n_work < 0 || n_list < 0 || batch < 1 || !counts || (n_work && !work) || (n_list && !ket_list)) return FJ_ERR_ARG;
+    if (out_work && (!out_parent || !out_kets)) return FJ_ERR_ARG;
+    long long items = 0, kets = 0;
+    for (int w = 0; w < n_work; ++w) {
+        const int* it = work + 4 * (size_t)w;
+        if ((it[2] >> 16) & 0xff) continue;
+        if (it[1] < 0 || it[3] < it[1] || it[3] > n_list) return FJ_ERR_ARG;
+        if (!out_work) {   // the most there can be
+            items += (it[3] - it[1] + batch - 1) / batch;
+            kets += it[3] - it[1];
+            continue;
+        }
+        const long long k0 = kets;
+        for (int e = it[1]; e < it[3]; ++e)
+            if (!((ket_list[e] >> 17) & 0x7f)) out_kets[kets++] = ket_list[e] & 0x1ffff;
+        const long long n = kets - k0, pieces = (n + batch - 1) / batch;
+        for (long long j = 0; j < pieces; ++j, ++items) {
+            int* o = out_work + 4 * items;
+            o[0] = it[0];
+            o[1] = (int)(k0 + j * n / pieces);
+            o[2] = it[2] & 0xffff;
+            o[3] = (int)(k0 + (j + 1) * n / pieces);
+            out_parent[items] = w;
+        }
+    }
+    counts[0] = items;
+    counts[1] = kets;
+    return 0;
+}

@@ -141,7 +141,7 @@ class CoopItems:
     ket_list: np.ndarray
     parent: np.ndarray
     parts: int
-    dev: tuple = ()           # (work, ket_list, identity) on the device
+    dev: tuple = ()           # (work, ket_list, identity where MIXED) on the device
     cover: tuple = ()         # MIXED: (offsets, planned items) of coop_cover
     tier: object = None       # MIXED: per-item tiers on the device, from the planned items'
 
@@ -152,19 +152,8 @@ def coop_items(work: np.ndarray, ket_list: np.ndarray, batch: int):
     chunk name its kets, and of the items of one bra pair's chunks the first
     lists every lane, so each quartet of the plan is taken once, whole. An
     item's kets are cut into equal pieces of at most `batch`."""
-    first = (ket_list & (0x7f << 17)) == 0
-    at = np.zeros(len(ket_list) + 1, dtype=np.int64)
-    np.cumsum(first, out=at[1:])
-    w = work.astype(np.int64)
-    parent = np.nonzero(((w[:, 2] >> 16) & 0xff) == 0)[0]
-    k0, n = at[w[parent, 1]], at[w[parent, 3]] - at[w[parent, 1]]
-    pieces = -(-n // batch)
-    rep = np.repeat(np.arange(len(parent)), pieces)
-    j = np.arange(len(rep)) - np.repeat(np.cumsum(pieces) - pieces, pieces)
-    lo = k0[rep] + j * n[rep] // pieces[rep]
-    hi = k0[rep] + (j + 1) * n[rep] // pieces[rep]
-    out = np.stack([w[parent[rep], 0], lo, w[parent[rep], 2] & 0xffff, hi], axis=1)
-    return out.astype(np.int32), (ket_list[first] & 0x1ffff).astype(np.int32), parent[rep].astype(np.int32)
+    from . import planner
+    return planner.coop_items(work, ket_list, batch)
 
 
 def coop_cover(work: np.ndarray, ket_list: np.ndarray, items):
@@ -182,10 +171,13 @@ def coop_cover(work: np.ndarray, ket_list: np.ndarray, items):
     if len(cut) or len(chunked):
         # the planned item (of the first bra chunk) and the item of an entry
         by_start = chunk0[np.argsort(w[chunk0, 1])]
-        by_first = np.argsort(cw[:, 1])
-        at = np.cumsum(lo == 0) - 1
-        under = lambda e: by_start[np.searchsorted(w[by_start, 1], e, side="right") - 1]       # noqa: E731
-        of_first = lambda e: by_first[np.searchsorted(cw[by_first, 1], at[e], side="right") - 1]   # noqa: E731
+        at = np.concatenate([[0], np.cumsum(lo == 0)])   # first chunks before an entry
+        under = lambda e: by_start[np.searchsorted(w[by_start, 1], e, side="right") - 1]   # noqa: E731
+
+        def of_first(e):   # in list order within a planned item, whose items are together
+            i = np.searchsorted(parent, under(e))
+            return np.searchsorted(cw[:, 1], cw[i, 1] + at[e] - at[w[parent[i], 1]], side="right") - 1
+
         plan = under(cut)
         # a later chunk is found by its quartet (bra, ket) among the cut first ones
         quartet = (w[plan, 0] << 17) | (ket_list[cut] & 0x1ffff)
@@ -389,7 +381,6 @@ class FockBuilder:
     # of the Coulomb and exchange blocks: J - K/2. Others (hjk.HJKBuild: J or K)
     # in the cooperative form alone; `launch` refuses them in any other.
     weights = (2.0, -0.5)
-
     def __init__(self, basis: Basis, D: np.ndarray, *, tau: float = 1e-12, threads=64,
                  mixed: bool = False, fp32_error: float = 1e-11, selector=None,
                  lane_flops=None, fp32_bound: float | None = None, planner: str = "auto",
@@ -860,11 +851,14 @@ class FockBuilder:
             return None
         # share the primitive quartets of an item over more workgroups while
         # there are few items and each has full passes to give
-        deg = np.concatenate([[0], np.cumsum(L.ket.deg[kets])])
-        most = int((L.bra.deg[work[:, 0]] * (deg[work[:, 3]] - deg[work[:, 1]])).max())
-        parts = max(1, min(COOP_GROUPS // len(work), -(-most // 256), 64))
+        parts = min(COOP_GROUPS // len(work), 64)
+        if parts > 1:
+            most = int((L.bra.deg[work[:, 0]] * np.add.reduceat(L.ket.deg[kets], work[:, 1])).max())
+            parts = min(parts, -(-most // 256))
+        parts = max(1, parts)
         c = CoopItems(work, kets, parent, parts)
-        c.dev = tuple(native.to_dev(x) for x in (work, kets, np.arange(len(work), dtype=np.int32)))
+        c.dev = (native.to_dev(work), native.to_dev(kets),
+                 native.to_dev(np.arange(len(work), dtype=np.int32)) if L.precision == MIXED else None)
         if L.precision == MIXED:
             c.cover = coop_cover(L.work, L.ket_list, (work, kets, parent))
         return c

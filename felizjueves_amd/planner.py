@@ -81,3 +81,18 @@ def plan_pairs(bra: Side, ket: Side, ket_table, systems: Systems, *, diag: int, 
     finally:
         native.lib().fj_plan_free(C.byref(res))
     return out, n_cold
+
+
+def coop_items(work: np.ndarray, ket_list: np.ndarray, batch: int):
+    """(work, ket list, parent) of planned items for the cooperative kernel
+    (fj_coop_items)."""
+    fn = native.lib().fj_coop_items
+    fn.restype = C.c_int
+    work, ket_list = (np.ascontiguousarray(x, dtype=np.int32) for x in (work, ket_list))
+    counts = (C.c_longlong * 2)()
+    p = lambda a: C.c_void_p(a.ctypes.data)   # noqa: E731
+    args = [p(work), C.c_int(len(work)), p(ket_list), C.c_int(len(ket_list)), C.c_int(batch)]
+    native.check(fn(*args, None, None, None, counts), "fj_coop_items")
+    out, parent, kets = (np.empty(s, dtype=np.int32) for s in ((counts[0], 4), counts[0], counts[1]))
+    native.check(fn(*args, p(out), p(parent), p(kets), counts), "fj_coop_items")
+    return out[:counts[0]], kets[:counts[1]], parent[:counts[0]]

@@ -153,6 +153,16 @@ int fj_plan_pairs(const FjPlanSide* bra, const FjPlanSide* ket, const int* mol_l
     double fp32_error, double fp32_bound, double est_scale, int threads, double lane_flops,
     double per_prim, double per_quartet, int max_prim, FjPlanResult* out);
 void fj_plan_free(FjPlanResult* out);
+/* The items of a planned launch for its cooperative kernel (fj_fc_; host
+ * code): of the planned items' lanes (ket, primitive chunk) those with a
+ * first chunk name their kets, and of the items of one bra pair's chunks the
+ * first lists every lane, so each quartet is taken once, whole; an item's
+ * kets are cut into equal pieces of at most `batch`.  out_work [n][4] (bra,
+ * first entry of out_kets, system, end entry), out_parent [n] the planned
+ * item, out_kets; counts[2]: n and the entries of out_kets.  out_work NULL:
+ * only upper bounds of the two. */
+int fj_coop_items(const int* work, int n_work, const int* ket_list, int n_list, int batch,
+    int* out_work, int* out_parent, int* out_kets, long long* counts);
 
 /* BEGIN F CLASSES (written by felizjueves_amd/gen_hip.py) */
 int fj_f_0000(fj_stream_t stream, int threads, int n_bra, int n_ket, int k_ab, int k_cd,
