@@ -381,6 +381,10 @@ class FockBuilder:
     # of the Coulomb and exchange blocks: J - K/2. Others (hjk.HJKBuild: J or K)
     # in the cooperative form alone; `launch` refuses them in any other.
     weights = (2.0, -0.5)
+    # Every build is for the first one's density (hjk.HJKBuild, staged for it):
+    # its block maxima are then formed once.
+    fixed_density = False
+
     def __init__(self, basis: Basis, D: np.ndarray, *, tau: float = 1e-12, threads=64,
                  mixed: bool = False, fp32_error: float = 1e-11, selector=None,
                  lane_flops=None, fp32_bound: float | None = None, planner: str = "auto",
@@ -1017,8 +1021,9 @@ class FockBuilder:
         main = stream if stream is not None else torch.cuda.current_stream()
         with torch.cuda.stream(main):
             self._F_flat.zero_()
-        for m, D in enumerate(D_devs):
-            native.density_blocks(self.shell_ao[m], self.shell_size[m], D, self.Dshs[m], main)
+        if not (self.fixed_density and getattr(self, "_built", False)):
+            for m, D in enumerate(D_devs):
+                native.density_blocks(self.shell_ao[m], self.shell_size[m], D, self.Dshs[m], main)
         if self.mixed:
             # every mixed launch's tiers, from this density, in one launch
             jobs = self._tier_jobs()

@@ -135,6 +135,23 @@ def _density(basis: Basis, D) -> np.ndarray:
     return D
 
 
+def _check(basis: Basis, tau: float, screen: str) -> None:
+    """What a split J / K stream of `basis` refuses."""
+    if screen not in SCREENS:
+        raise ValueError(f"screen = {screen!r} is not one of {SCREENS}")
+    if not (isinstance(tau, (int, float)) and not isinstance(tau, bool) and math.isfinite(tau)
+            and tau >= 0.0):
+        raise ValueError(f"tau = {tau!r} is not a finite float >= 0")
+    if basis.l_max > SPLIT_LMAX:
+        raise ValueError(f"shells up to l = {basis.l_max}: the split kernels are built through "
+                         f"l = {SPLIT_LMAX}")
+    deg = np.outer(basis.shell_nprim, basis.shell_nprim)
+    if deg.size and deg.max() > MAX_PRIM_PAIRS:
+        a, b = np.argwhere(deg > MAX_PRIM_PAIRS)[0]
+        raise ValueError(f"shell pair ({a}, {b}) has degree {deg[a, b]} > MAX_PRIM_PAIRS = "
+                         f"{MAX_PRIM_PAIRS}, the kernels' staging cap")
+
+
 # default sub-pair size: at most 2 x 2 primitive quartets per lane. Measured
 # on the GPU (J of the three-atom s,s,p,d system / the 10-atom cluster, ms):
 # whole pairs 3,182 / 16,797; 16: 1,042 / 7,539; 9: 483 / 3,721;
@@ -157,14 +174,7 @@ def hjk_launches(basis: Basis, D, *, tau: float, mode: str = "canonical",
     the quartet's (each through its own FP64 HRR and atomics)."""
     if mode not in MODES:
         raise ValueError(f"mode = {mode!r}: only the canonical class mode is built ({MODES})")
-    if screen not in SCREENS:
-        raise ValueError(f"screen = {screen!r} is not one of {SCREENS}")
-    if not (isinstance(tau, (int, float)) and not isinstance(tau, bool) and math.isfinite(tau)
-            and tau >= 0.0):
-        raise ValueError(f"tau = {tau!r} is not a finite float >= 0")
-    if basis.l_max > SPLIT_LMAX:
-        raise ValueError(f"shells up to l = {basis.l_max}: the split kernels are built through "
-                         f"l = {SPLIT_LMAX}")
+    _check(basis, tau, screen)
     D = _density(basis, D)
     ns = basis.n_sh
     by_cls: dict = {}
@@ -177,12 +187,8 @@ def hjk_launches(basis: Basis, D, *, tau: float, mode: str = "canonical",
         pp = P.primitive_pairs(basis, sps)
         for k, (a, b) in enumerate(sps):
             g = pp.bound[pp.pair == k]
-            deg = len(g)
-            if deg > MAX_PRIM_PAIRS:
-                raise ValueError(f"shell pair ({a}, {b}) has degree {deg} > MAX_PRIM_PAIRS = "
-                                 f"{MAX_PRIM_PAIRS}, the kernels' staging cap")
             G[a, b] = math.fsum(g)
-            pairs.append(HPair(a, b, la, lb, deg, G[a, b]))
+            pairs.append(HPair(a, b, la, lb, len(g), G[a, b]))
     pairs.sort(key=lambda p: (p.a, p.b))            # pair order: a outer, b inner
     bins: dict = {}
     for p in pairs:
@@ -372,10 +378,12 @@ class HJKBuild:
     def __init__(self, basis: Basis, D, *, tau: float = 1e-12, screen: str = "j",
                  threads: int = 64, plan: HPlan | None = None):
         from . import native
-        D = _density(basis, D)
-        self.plan = plan if plan is not None else hjk_launches(basis, D, tau=tau, screen=screen)
-        if self.plan.screen != screen:
+        if plan is None:
+            _check(basis, tau, screen)
+        elif plan.screen != screen:
             raise ValueError("the plan is for the other screen")
+        D = _density(basis, D)
+        self._plan, self._args = plan, (basis, D, tau)
         self.basis, self.screen, self.threads = basis, screen, threads
         self.kind = "hj" if screen == "j" else "hk"
         self.graph = None
@@ -392,12 +400,22 @@ class HJKBuild:
                 self._stage(D)
                 return
             self.builder.weights = (2.0, 0.0) if screen == "j" else (0.0, 1.0)
+            self.builder.fixed_density = True
             self.quartets_computed, self.flops = self.builder.n_quartets, self.builder.flops
             self.builder.to_device()
             self._D = native.to_dev(np.ascontiguousarray(D))
             self.X = self.builder.F
             return
         self._stage(D)
+
+    @property
+    def plan(self) -> HPlan:
+        """The split stream: the given plan, else the default one, planned when
+        it is asked for (a build without a plan does not run it)."""
+        if self._plan is None:
+            basis, D, tau = self._args
+            self._plan = hjk_launches(basis, D, tau=tau, screen=self.screen)
+        return self._plan
 
     def _stage(self, D) -> None:
         """Every launch's arguments on the device (a given plan)."""

@@ -209,3 +209,29 @@ def test_split_build_counts_what_it_runs(monkeypatch):
     monkeypatch.setattr(hjk, "GpuHJKRunner", lambda: type("R", (), {"zeros": lambda self, n: None})())
     b = hjk.HJKBuild(fx.basis, fx.density, tau=0.0, plan=hjk.hjk_launches(fx.basis, fx.density, tau=0.0))
     assert b.quartets_computed == n ** 4 and b.builder is None
+
+
+def test_split_build_plans_the_ordered_stream_when_asked(monkeypatch):
+    """Without a plan the ordered stream is not planned until `plan` is read;
+    what the stream refuses is refused all the same, before and at once."""
+    from felizjueves_amd import fock, native
+    from felizjueves_amd.basis import Basis
+    fx = load_fixture("h2o_sto3g")
+    monkeypatch.setattr(fock.FockBuilder, "to_device", lambda self: setattr(self, "F", None))
+    monkeypatch.setattr(native, "to_dev", lambda x: x)
+    planned, launches = [], hjk.hjk_launches
+    monkeypatch.setattr(hjk, "hjk_launches", lambda *a, **k: planned.append(1) or launches(*a, **k))
+    b = hjk.HJKBuild(fx.basis, fx.density, screen="k")
+    assert not planned and len(b.plan) == len(launches(fx.basis, fx.density, tau=1e-12, screen="k")) == len(b.plan)
+    assert planned == [1] and b.plan.screen == "k"
+    n = 12   # one shell of 12 primitives: 144 pairs
+    deep = Basis.from_arrays(np.array([0]), np.zeros((1, 3)), np.array([n]), 0.1 * 1.5 ** np.arange(n), np.full(n, 0.2))
+    for kw in (dict(tau=-1.0), dict(tau=float("nan")), dict(screen="x")):
+        with pytest.raises(ValueError):
+            hjk.HJKBuild(fx.basis, fx.density, **kw)
+    with pytest.raises(ValueError, match="degree 144"):
+        hjk.HJKBuild(deep, np.eye(1))
+    with pytest.raises(ValueError, match="degree 144"):
+        launches(deep, np.eye(1), tau=0.0)
+    with pytest.raises(ValueError, match="l = 3"):
+        hjk.HJKBuild(load_fixture("co_ccpvtz").basis, load_fixture("co_ccpvtz").density)
