@@ -304,9 +304,10 @@ __global__ void __launch_bounds__(DQ_THREADS, (LA + LB >= 5 ? 1 : 2)) fj_dfquad_
             }
             fj_wave_sync();   // before the next tables
         }
-        // the wavefronts' sums, in turn into the first's
+        // the wavefronts' sums, in turn into the first's (a wavefront past the
+        // bra's primitives has none)
         double* const sum = &S.t[0][0];
-        for (int w = 1; w < DQ_WAVES; ++w) {
+        for (int w = 1; w < min(DQ_WAVES, i1 - i0); ++w) {   // uniform over the workgroup
             __syncthreads();
             if (wave == w) {
 #pragma unroll
