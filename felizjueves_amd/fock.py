@@ -304,6 +304,9 @@ def orient_pairs(basis: Basis, pairs: list) -> list:
         near_b = dB < dA
         size = np.abs(p.rec[:, 7]) * (2.0 * z) ** (-0.5 * (p.la + p.lb))
         tot = size.sum()
+        if not tot > 0.0:   # every record vanished (far, tight shells): nothing to amplify
+            out.append(p)
+            continue
         amp_on_a = (1.0 + dA * np.sqrt(2.0 * z)) ** p.lb     # built on A
         amp_on_b = (1.0 + dB * np.sqrt(2.0 * z)) ** p.la     # built on B
         err_a = (size * amp_on_a)[near_b].sum() / tot

@@ -235,3 +235,21 @@ def test_split_build_plans_the_ordered_stream_when_asked(monkeypatch):
         launches(deep, np.eye(1), tau=0.0)
     with pytest.raises(ValueError, match="l = 3"):
         hjk.HJKBuild(load_fixture("co_ccpvtz").basis, load_fixture("co_ccpvtz").density)
+
+
+def test_split_build_of_pairs_that_vanish(monkeypatch):
+    """Tight shells far apart: their pair's records underflow to zero, and the
+    build without a plan takes them (at tau = 0 no pair is dropped)."""
+    from felizjueves_amd import fock, native
+    from felizjueves_amd.basis import Basis
+    monkeypatch.setattr(fock.FockBuilder, "to_device", lambda self: setattr(self, "F", None))
+    monkeypatch.setattr(native, "to_dev", lambda x: x)
+    basis = Basis.from_arrays(np.array([0, 1, 2]), np.array([[0.0, 0, 0], [0, 0, 9.0], [0, 9.0, 0]]), np.array([1, 2, 1]),
+                              np.array([3e4, 2e4, 9e3, 5e3]), np.array([1.0, 0.5, 0.7, 1.0]))
+    D = np.eye(basis.n_ao)
+    for tau in (0.0, 1e-12):
+        b = hjk.HJKBuild(basis, D, tau=tau)
+        pairs = [p for t in b.builder.tables.values() for p in t.pairs]
+        assert all(p.degree == len(p.rec) > 0 for p in pairs)
+        assert tau > 0 or len(pairs) == 6
+        assert tau > 0 or min(np.abs(p.rec[:, 7]).max() for p in pairs) == 0.0
