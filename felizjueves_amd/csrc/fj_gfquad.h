@@ -30,12 +30,12 @@
 // multiplied by a zero A operand (the summed index).
 //
 // Measured on MI355X, every class of the s,s,p,d 8-atom gradient alone (29.8
-// million primitive quartets): 666 ms in the loop form, 55 ms here, and 22.3
-// -> 6.4 ms for the three-atom one; e.g. (dd|dd) 32.2 -> 4.8 ms, (sp|dd) 75.8
-// -> 2.8 ms, (ss|sp) 4.8 -> 1.1 ms. The matrix cores are busy 13 to 26% of the
+// million primitive quartets): 666 ms in the loop form, 54 ms here, and 22.3
+// -> 3.0 ms for the three-atom one; e.g. (dd|dd) 32.2 -> 4.8 ms, (sp|dd) 75.8
+// -> 2.8 ms, (ss|sp) 4.8 -> 1.1 ms. The matrix cores are busy 11 to 27% of the
 // time of the classes with a d shell in the ket; to each matrix step come 8 to
-// 39 VALU instructions of the towers and the last stage (12.5 at (dd|dd)), and
-// the wavefronts wait in 15 to 28% of their cycles.
+// 44 VALU instructions of the towers and the last stage (9 at (dd|dd)), and the
+// wavefronts wait in 14 to 28% of their cycles.
 //
 // The includer provides fj_device.h (the device one, or the CPU emulation)
 // and fj_gfloop.h.

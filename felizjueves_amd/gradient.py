@@ -124,7 +124,7 @@ def gf_launches(basis: Basis, shell_atom) -> GfStream:
 def default_threads(cls) -> int:
     """Workgroup size of a class: 256 lanes, the width of the matrix-core
     kernel (fj_gfquad.h); narrower ones run the loop form (the three-atom
-    s,s,p,d gradient, classes one after another: 6.1 ms against 22 ms)."""
+    s,s,p,d gradient, classes one after another: 3.0 ms against 22 ms)."""
     return 256
 
 
